@@ -24,8 +24,8 @@
 //     per tile before the main loop (the reference's fp16 semantics); raw path
 //     -- exact fp32 v_mfma_f32_32x32x2_f32 on (dmin*m, -(xd*xsum)) per stage.
 //   * Blocks are mapped XCD-major: block b runs on XCD b % 8, and each XCD gets
-//     a contiguous range of tiles (token tiles fastest) so the tiles that share
-//     a weight panel share one L2.
+//     a contiguous range of tiles, ordered (tile_at) so that the tiles resident
+//     at once share weight panels and token tiles through one L2.
 #include "bq_device.hpp"
 #include "bq_internal.hpp"
 
@@ -45,13 +45,38 @@ struct TileMap {
     int mt, nt;  // token tile, weight-row tile (over concatenated parts)
 };
 
+// Order of the tiles: an XCD's resident workgroups (64 of the 128-token tiles,
+// 96 of the 32-token ones) run consecutive indices at about the same K stage,
+// so the fewer bytes of weight panels and token tiles those cover, the more of
+// every stage its 4 MB L2 serves.  With more token tiles than one such round
+// wants, the order walks G panels per token tile instead of all token tiles of
+// one panel: G = 8 at 128 tokens (64 indices = 8 panels x 8 token tiles of 18 +
+// 16 KB a stage; panel-major 8192 rows: 1 x 64, 1 MB of tokens a stage from
+// beyond the L2), G = 4 at 32 tokens (18 and 4 KB: 4 x 24).  Up to kRound token
+// tiles the panel-major order is already as compact (512 rows as 32-token tiles,
+// 14336 x 2560: 66.4 us, in groups of 8 70.1).  9216 x 3072 W144: 8192 rows
+// 642 -> 606 us, 2048 rows 166.6 -> 162.2 (G = 4 / 16 1-2% behind at 8192 rows).
+template <int TM>
+BQ_DEV void tile_at(int idx, int ntm, int ntn, TileMap& t) {
+    constexpr int G = TM == 32 ? 4 : 8, kRound = TM == 32 ? 24 : 8;
+    if (ntm <= kRound) {
+        t.mt = idx % ntm;
+        t.nt = idx / ntm;
+        return;
+    }
+    const int grp = idx / (G * ntm), first = grp * G;
+    const int width = min(G, ntn - first), r = idx - first * ntm;
+    t.mt = r / width;
+    t.nt = first + r % width;
+}
+
+template <int TM>
 BQ_DEV bool map_tile(int b, int ntm, int ntn, TileMap& t) {
     const int ntiles = ntm * ntn;
     const int per = (ntiles + kXcds - 1) / kXcds;
     const int idx = (b % kXcds) * per + b / kXcds;
     if (idx >= ntiles) return false;
-    t.mt = idx % ntm;
-    t.nt = idx / ntm;
+    tile_at<TM>(idx, ntm, ntn, t);
     return true;
 }
 
@@ -73,18 +98,18 @@ struct TailSplit {
 // Block -> (tile, slice, slices).  Returns false for a block with no work.
 // XCD-major over the whole tiles as map_tile; a leftover tile's k slices are
 // consecutive blocks.
+template <int TM>
 BQ_DEV bool map_tile_tail(int b, int ntm, int ntn, const TailSplit& ts, TileMap& t, int& kc, int& ks, int& left) {
     left = -1;
     if (ts.k <= 1) {
         kc = blockIdx.y;
-        return map_tile(b, ntm, ntn, t);
+        return map_tile<TM>(b, ntm, ntn, t);
     }
     if (b < ts.gridfull) {
         const int per = ts.gridfull / kXcds;
         const int idx = (b % kXcds) * per + b / kXcds;
         if (idx >= ts.nfull) return false;
-        t.mt = idx % ntm;
-        t.nt = idx / ntm;
+        tile_at<TM>(idx, ntm, ntn, t);
         kc = 0;
         ks = 1;
         return true;
@@ -95,8 +120,7 @@ BQ_DEV bool map_tile_tail(int b, int ntm, int ntn, const TailSplit& ts, TileMap&
     kc = j % ts.k;
     ks = ts.k;
     const int idx = ts.nfull + left;
-    t.mt = idx % ntm;
-    t.nt = idx / ntm;
+    tile_at<TM>(idx, ntm, ntn, t);
     return true;
 }
 
@@ -219,7 +243,7 @@ k_mmq_q5k_raw(PartTable pt, int ntm, int ntn, int rows, int K, const int8_t* __r
     __shared__ __attribute__((aligned(16))) Smem<TM> sm;
     TileMap tm;
     int kc, left;
-    if (!map_tile_tail(blockIdx.x, ntm, ntn, ts, tm, kc, ksplit, left)) return;
+    if (!map_tile_tail<TM>(blockIdx.x, ntm, ntn, ts, tm, kc, ksplit, left)) return;
     int nbase = tm.nt * kTN;
     const int p = part_of_ntile(pt, nbase);
     const int Nloc = pt.N[p];
@@ -634,7 +658,7 @@ k_mmq_w144(PartTable pt, int ntm, int ntn, int rows, int K, const int8_t* __rest
     __shared__ __attribute__((aligned(16))) SmemStage<TM> sm1;
     TileMap tm;
     int kc, left;
-    if (!map_tile_tail(blockIdx.x, ntm, ntn, ts, tm, kc, ksplit, left)) return;
+    if (!map_tile_tail<TM>(blockIdx.x, ntm, ntn, ts, tm, kc, ksplit, left)) return;
     int nbase = tm.nt * kTN;
     const int p = part_of_ntile(pt, nbase);
     const int Nloc = pt.N[p];
@@ -754,17 +778,18 @@ k_mmq_w144(PartTable pt, int ntm, int ntn, int rows, int K, const int8_t* __rest
 // y of the leftover tiles = the sum of their k slices (fixed slice order), one
 // float4 per thread: thread i -> tile i / (TM * 32), token row, 4 columns
 template <int TM>
-__global__ void __launch_bounds__(256) k_sum_tail(const float* __restrict__ ws, PartTable pt, int ntm, int rows,
-                                                  TailSplit ts) {
+__global__ void __launch_bounds__(256) k_sum_tail(const float* __restrict__ ws, PartTable pt, int ntm, int ntn,
+                                                  int rows, TailSplit ts) {
     const size_t per = (size_t)TM * (kTN / 4);
     const size_t i = (size_t)blockIdx.x * 256 + threadIdx.x;
     if (i >= per * ts.nleft) return;
     const int left = (int)(i / per);
     const int e = (int)(i % per), ml = e / (kTN / 4), c4 = e % (kTN / 4);
-    const int idx = ts.nfull + left;
-    const int m = (idx % ntm) * TM + ml;
+    TileMap t;
+    tile_at<TM>(ts.nfull + left, ntm, ntn, t);
+    const int m = t.mt * TM + ml;
     if (m >= rows) return;
-    int nbase = (idx / ntm) * kTN;
+    int nbase = t.nt * kTN;
     const int p = part_of_ntile(pt, nbase);
     const size_t slice = (size_t)ts.nleft * kTN * TM;
     const f32x4* src = (const f32x4*)(ws + (size_t)left * kTN * TM) + e;
@@ -885,7 +910,7 @@ k_mmq_q6k_dma(PartTable pt, int ntm, int ntn, int rows, int K, const int8_t* __r
     __shared__ __attribute__((aligned(16))) SmemQ6Stage<TM> sm0;
     __shared__ __attribute__((aligned(16))) SmemQ6Stage<TM> sm1;
     TileMap tm;
-    if (!map_tile(blockIdx.x, ntm, ntn, tm)) return;
+    if (!map_tile<TM>(blockIdx.x, ntm, ntn, tm)) return;
     int nbase = tm.nt * kTN;
     const int p = part_of_ntile(pt, nbase);
     const int Nloc = pt.N[p];
@@ -1156,7 +1181,7 @@ static hipError_t launch_w144_tm(const PartTable& pt, int ntm, int ntn, int ks, 
                       xq, xd, xsum, xdh, 1, ws, ts);
         const size_t n4 = (size_t)ts.nleft * TM * (kTN / 4);
         launch_kernel(k_sum_tail<TM>, dim3((unsigned)((n4 + 255) / 256)), dim3(256), 0, st, (const float*)ws, pt,
-                      ntm, rows, ts);
+                      ntm, ntn, rows, ts);
         return hipGetLastError();
     }
     const dim3 grid(mmq_grid(ntm, ntn).x, ks);
@@ -1189,7 +1214,7 @@ static hipError_t launch_raw_tm(const PartTable& pt, int ntm, int ntn, int ks, c
                       K, xq, xd, xsum, 1, ws, ts);
         const size_t n4 = (size_t)ts.nleft * TM * (kTN / 4);
         launch_kernel(k_sum_tail<TM>, dim3((unsigned)((n4 + 255) / 256)), dim3(256), 0, st, (const float*)ws, pt,
-                      ntm, rows, ts);
+                      ntm, ntn, rows, ts);
         return hipGetLastError();
     }
     const dim3 grid(mmq_grid(ntm, ntn).x, ks);
