@@ -32,6 +32,7 @@
 #include <stdlib.h>
 
 #include <algorithm>
+#include <cmath>
 
 namespace bq {
 
@@ -70,13 +71,37 @@ BQ_DEV void tile_at(int idx, int ntm, int ntn, TileMap& t) {
     t.nt = first + r % width;
 }
 
+// Block b of a launch of ntm x ntn tiles in ks K slices -> (tile, slice kc).
+// The ntiles * ks pieces, a tile's slices next to each other, are dealt to the
+// XCDs in equal contiguous ranges (block b runs on XCD b % 8), so an XCD holds
+// at most one piece more than another; inside an XCD the blocks go slice by
+// slice, so that the first slices, which hold the W144 min term, start first and
+// on a CU each (two of them on one CU: 7040 x 5120 at 41 rows 21.9 -> 28.5 us).
+// (With the slices on blockIdx.y each XCD took ceil(ntiles / 8) tiles times
+// ks: Q6_K 2560 x 7168 at 640 rows, 100 tiles x 5 slices, put 65 workgroups on an
+// XCD's 64 slots: 97 us, now 67.  No block of a range may be empty: with 7 empty
+// ones in front of 63 the same call took 93.)
 template <int TM>
-BQ_DEV bool map_tile(int b, int ntm, int ntn, TileMap& t) {
-    const int ntiles = ntm * ntn;
-    const int per = (ntiles + kXcds - 1) / kXcds;
-    const int idx = (b % kXcds) * per + b / kXcds;
-    if (idx >= ntiles) return false;
-    tile_at<TM>(idx, ntm, ntn, t);
+BQ_DEV bool map_tile(int b, int ntm, int ntn, int ks, TileMap& t, int& kc) {
+    const int n = ntm * ntn * ks, per = (n + kXcds - 1) / kXcds;
+    const int p0 = (b % kXcds) * per, p1 = min(p0 + per, n);
+    int j = b / kXcds;
+    kc = 0;
+    if (p0 + j >= p1) return false;
+    if (ks == 1) {
+        tile_at<TM>(p0 + j, ntm, ntn, t);
+        return true;
+    }
+    // the j-th piece of [p0, p1) in the order of (slice, tile)
+    const int lead = p0 % ks;
+    int first;
+    for (;; ++kc) {
+        first = p0 + (kc >= lead ? kc - lead : kc - lead + ks);
+        const int c = first < p1 ? (p1 - 1 - first) / ks + 1 : 0;
+        if (j < c) break;
+        j -= c;
+    }
+    tile_at<TM>(first / ks + j, ntm, ntn, t);
     return true;
 }
 
@@ -87,7 +112,7 @@ BQ_DEV bool map_tile(int b, int ntm, int ntn, TileMap& t) {
 // k K slices, so the leftover work spreads over L * k pieces; the slices'
 // partial tiles go to the caller's workspace [slice][leftover tile][TM][128]
 // and k_sum_tail adds them in slice order.  k == 1: no tail split (the
-// uniform K split, blockIdx.y, or no split at all).
+// uniform K split or no split at all).
 struct TailSplit {
     int k = 1;        // slices per leftover tile
     int nfull = 0;    // tiles run whole (tile indices 0 .. nfull-1)
@@ -101,10 +126,7 @@ struct TailSplit {
 template <int TM>
 BQ_DEV bool map_tile_tail(int b, int ntm, int ntn, const TailSplit& ts, TileMap& t, int& kc, int& ks, int& left) {
     left = -1;
-    if (ts.k <= 1) {
-        kc = blockIdx.y;
-        return map_tile<TM>(b, ntm, ntn, t);
-    }
+    if (ts.k <= 1) return map_tile<TM>(b, ntm, ntn, ks, t, kc);
     if (b < ts.gridfull) {
         const int per = ts.gridfull / kXcds;
         const int idx = (b % kXcds) * per + b / kXcds;
@@ -144,7 +166,7 @@ BQ_DEV int part_of_ntile(const PartTable& pt, int& nbase) {
 }
 
 // Token-tile height TM of the prefill kernels (128 or 32, chosen per launch
-// by mmq_tile_rows): the weight tile stays 128 rows, the
+// by mmq_pick): the weight tile stays 128 rows, the
 // four waves form a WN x WM grid of (NT x 32) x (MT x 32) sub-tiles (TM 128:
 // 2 x 2 waves of 64 x 64; TM 32: 4 x 1 waves of 32 x 32).
 template <int TM>
@@ -910,7 +932,8 @@ k_mmq_q6k_dma(PartTable pt, int ntm, int ntn, int rows, int K, const int8_t* __r
     __shared__ __attribute__((aligned(16))) SmemQ6Stage<TM> sm0;
     __shared__ __attribute__((aligned(16))) SmemQ6Stage<TM> sm1;
     TileMap tm;
-    if (!map_tile<TM>(blockIdx.x, ntm, ntn, tm)) return;
+    int kc;
+    if (!map_tile<TM>(blockIdx.x, ntm, ntn, ksplit, tm, kc)) return;
     int nbase = tm.nt * kTN;
     const int p = part_of_ntile(pt, nbase);
     const int Nloc = pt.N[p];
@@ -936,8 +959,7 @@ k_mmq_q6k_dma(PartTable pt, int ntm, int ntn, int rows, int K, const int8_t* __r
     o.s_off = (uint32_t)(lane >> 1) * row_bytes + 128u + 16u * (uint32_t)(lane & 1);
     o.xd_off = (uint32_t)lane * (uint32_t)(nb * 4);
 
-    // K split (blockIdx.y of ksplit): stage pairs [s0, s1) of this slice
-    const int kc = blockIdx.y;
+    // K split (slice kc of ksplit): stage pairs [s0, s1) of this slice
     const int s0 = 2 * (kc * (nst / 2) / ksplit), s1 = 2 * ((kc + 1) * (nst / 2) / ksplit);
     q6_dma<TM>(sm0, wstage(s0), row_bytes, xq, xd, o, m0, rows, K, nb, s0, wave, lane);
     const MfmaCvt cv = mfma_cvt_init(lane);
@@ -997,11 +1019,8 @@ static int ntotal(const PartTable& pt) {
     return n;
 }
 
-static dim3 mmq_grid(int ntm, int ntn) {
-    const int ntiles = ntm * ntn;
-    const int per = (ntiles + kXcds - 1) / kXcds;
-    return dim3(per * kXcds);
-}
+// blocks of map_tile's deal (equal ranges of the XCDs)
+static dim3 mmq_grid(int ntm, int ntn, int ks) { return dim3((ntm * ntn * ks + kXcds - 1) / kXcds * kXcds); }
 
 // K split.  A launch with fewer tiles than the workgroup slots (two per CU
 // for the 128-token tiles, three for the 32-token tiles; 512 / 768 on
@@ -1029,49 +1048,75 @@ int mmq_ksplit(int rows, int K, int ntot, bool stage_units, size_t ws_floats, in
     return (units + per - 1) / per;
 }
 
-// Token-tile height (128 or 32) of the DMA-staged kernels for a launch: the
-// one with the smaller estimated work on the busiest CU, ceil(workgroups /
-// CUs) x tile height x the longest K slice, the 32-token tile's work
-// weighted by e32 (its cost per output relative to the 128-token tile on a
-// full GPU, measured at 4096 rows: W144 1.115, Q6_K 1.06, raw Q5_K 1.33 --
-// its in-kernel unpack of the weight tile is shared by a quarter of the
-// tokens).  Short calls take
-// the 32-token tile (the 128-token tile costs the same at any row count up
-// to 128); at a few hundred to a few thousand rows it depends on how evenly
-// the tiles fill the workgroup slots.
 TailSplit mmq_tail_split(int ntiles, int units, size_t ws_floats, int tm, float e, int cus);
 constexpr float kTailMinSaving = 192.f;  // see mmq_tail_split
-// the fixed cost of a split launch (its summing launch and partial-tile
-// traffic, about 8 us) in the tile-height estimate's units
-constexpr float kSplitCost = 384.f;
 
-// tail: the kernel takes the leftover-tile split (both Q5_K tiers), so the
-// busiest CU's count is the split one
-int mmq_tile_rows(int rows, int K, int ntot, bool stage_units, size_t ws_floats, float e32, bool tail, int cus) {
-    float best = 0.f;
-    int pick = 128;
+// Token-tile height (128 or 32) and K split of a launch: the pair with the
+// smallest estimated time
+//   start[tm] + stages per slice x c[tm] x load + 2.5 us if a sum launch follows,
+// c = us per 128-value stage and workgroup per CU of a full GPU.  load: the
+// workgroups of the busiest CU (per XCD, as they are dealt), with two corrections.
+// A CU that holds a single 128-token tile takes 1.05 (one wave per SIMD keeps
+// it nearly as busy as two), one that holds two no less than `pair` = 1.6
+// (W144, unsplit) to 1.9 loads' time; the 32-token tile 1.3 and 1.9.  With the
+// leftover-tile split the load is the split one.  Fitted to both heights at
+// every split, 9 shapes x 11 row counts (9216 / 14336 / 8704 x 2560 / 3072 and
+// 2560 x 4096 W144, raw 3072 x 4096, Q6_K 3072 x 9216 and 2560 x 7168; 16..2048
+// rows).  Against the estimate this replaces (tile height weighted by 1.06 ..
+// 1.33, always the largest split): 14336 x 2560 at 512 rows 68.1 -> 59.7 us
+// (128 tokens instead of 32), 9216 x 3072 at 768 rows 78.8 -> 69.2, 8704 x 2560 at 768 /
+// 128 rows 66.3 -> 57.8 / 27.6 -> 24.5, 2560 x 4096 at 1536 rows 66.6 -> 58.1,
+// raw 3072 x 4096 at 300 rows 37.1 -> 32.9.
+struct TileCost {
+    float c128, c32, pair;
+    bool tail;   // the kernel takes the leftover-tile split
+    float e32;   // its 32-token tile's cost per output over the 128-token one's
+};
+constexpr TileCost kCostW144 = {1.40f, 0.425f, 1.62f, true, 1.115f};
+constexpr TileCost kCostRaw = {2.02f, 0.62f, 1.92f, true, 1.33f};
+constexpr TileCost kCostQ6 = {2.4f, 0.64f, 1.9f, false, 1.f};
+constexpr float kSplitUs = 2.5f, kStartUs128 = 11.5f, kStartUs32 = 9.f;
+
+struct TilePick {
+    int tm, ks;
+    TailSplit ts;
+};
+
+TilePick mmq_pick(int rows, int K, int ntot, bool stage_units, size_t ws_floats, const TileCost& tc, int cus) {
+    TilePick best = {128, 1, {}};
+    float best_us = -1.f;
+    const int units = stage_units ? K >> 7 : K >> 8;
     for (const int tm : {128, 32}) {
-        const int ks = mmq_ksplit(rows, K, ntot, stage_units, ws_floats, tm, cus);
-        const long long ctas = (long long)((rows + tm - 1) / tm) * (ntot / kTN) * ks;
-        const int units = stage_units ? K >> 7 : K >> 8;
-        const int per = (units + ks - 1) / ks;
-        float load = (float)((ctas + cus - 1) / cus);
-        bool split = ks > 1;
-        if (tail && ks == 1) {
-            const TailSplit ts = mmq_tail_split((int)ctas, units, ws_floats, tm, tm == 32 ? e32 : 1.f, cus);
-            if (ts.k > 1) {
-                load = (float)(ctas / cus) + (float)((ts.nleft * ts.k + cus - 1) / cus) / (float)ts.k;
-                split = true;
+        const int ntiles = ((rows + tm - 1) / tm) * (ntot / kTN);
+        const int ksmax = mmq_ksplit(rows, K, ntot, stage_units, ws_floats, tm, cus);
+        const float lone = tm == 128 ? 1.05f : 1.3f;
+        for (int k = 1; k <= ksmax; ++k) {
+            const int per = (units + k - 1) / k;
+            if ((units + per - 1) / per != k) continue;  // fewer slices have the same longest one
+            const float l = (float)((ntiles * k + kXcds - 1) / kXcds) * (float)kXcds / (float)cus;
+            const float pair = tm == 128 && k == 1 ? tc.pair : 1.9f;
+            float load;
+            if (l <= 1.f)
+                load = lone;
+            else if (l <= 2.f)
+                load = std::max(l, pair);
+            else if (tm == 32)  // up to three at once, then one after another as slots free up
+                load = l <= 3.f ? 2.45f + 0.35f * (l - 2.f) : l + 0.3f;
+            else  // two at once: nearly whole rounds
+                load = std::min(std::ceil(l) + 0.05f, l + 0.6f);
+            TailSplit ts;
+            if (tc.tail && k == 1) ts = mmq_tail_split(ntiles, units, ws_floats, tm, tm == 32 ? tc.e32 : 1.f, cus);
+            if (ts.k > 1) load = (float)(ntiles / cus) + (float)((ts.nleft * ts.k + cus - 1) / cus) / (float)ts.k;
+            const float stage = (float)(stage_units ? per : 2 * per) * (tm == 128 ? tc.c128 : tc.c32);
+            const float extra = k > 1 ? kSplitUs : 0.f;
+            const float us = (tm == 128 ? kStartUs128 : kStartUs32) + stage * load + extra;
+            if (best_us < 0.f || us < best_us) {
+                best_us = us;
+                best = {tm, k, ts};
             }
         }
-        // a split launch also pays its summing launch and partial-tile traffic
-        const float est = load * tm * per * (tm == 32 ? e32 : 1.f) + (split ? kSplitCost : 0.f);
-        if (tm == 128 || est < best) {
-            best = est;
-            pick = tm;
-        }
     }
-    return pick;
+    return best;
 }
 
 // y_p = sum over the K slices of the workspace (fixed order), 4 floats per
@@ -1184,7 +1229,7 @@ static hipError_t launch_w144_tm(const PartTable& pt, int ntm, int ntn, int ks, 
                       ntm, ntn, rows, ts);
         return hipGetLastError();
     }
-    const dim3 grid(mmq_grid(ntm, ntn).x, ks);
+    const dim3 grid = mmq_grid(ntm, ntn, ks);
     launch_kernel(k_mmq_w144<TM, XI>, grid, dim3(256), 0, st, pt, ntm, ntn, rows, K, xq, xd, xsum, xdh, ks, ws, ts);
     if (ks > 1) return sum_splits(pt, ks, rows, ws, st);
     return hipGetLastError();
@@ -1193,13 +1238,10 @@ static hipError_t launch_w144_tm(const PartTable& pt, int ntm, int ntn, int ks, 
 hipError_t launch_mmq_q5k_144(PartTable pt, int rows, int K, const int8_t* xq, const float* xd,
                               const int32_t* xsum, uint16_t* xdh, hipStream_t st, int cus, float* ws,
                               size_t ws_floats) {
-    const int tm = mmq_tile_rows(rows, K, ntotal(pt), false, ws ? ws_floats : 0, 1.115f, true, cus);
+    const auto [tm, ks, ts] = mmq_pick(rows, K, ntotal(pt), false, ws ? ws_floats : 0, kCostW144, cus);
     const int ntm = (rows + tm - 1) / tm;
     const int ntn = ntile_count(pt);
     if (ntm == 0 || ntn == 0) return hipSuccess;
-    const int ks = mmq_ksplit(rows, K, ntotal(pt), false, ws ? ws_floats : 0, tm, cus);
-    const TailSplit ts = ks > 1 ? TailSplit{}
-                                : mmq_tail_split(ntm * ntn, K >> 8, ws ? ws_floats : 0, tm, tm == 32 ? 1.115f : 1.f, cus);
     if (tm == 32 && rows <= kXdhInlineRows)
         return launch_w144_tm<32, true>(pt, ntm, ntn, ks, ts, rows, K, xq, xd, xsum, xdh, st, ws);
     if (tm == 32) return launch_w144_tm<32, false>(pt, ntm, ntn, ks, ts, rows, K, xq, xd, xsum, xdh, st, ws);
@@ -1217,7 +1259,7 @@ static hipError_t launch_raw_tm(const PartTable& pt, int ntm, int ntn, int ks, c
                       ntm, ntn, rows, ts);
         return hipGetLastError();
     }
-    const dim3 grid(mmq_grid(ntm, ntn).x, ks);
+    const dim3 grid = mmq_grid(ntm, ntn, ks);
     launch_kernel(k_mmq_q5k_raw<TM>, grid, dim3(256), 0, st, pt, ntm, ntn, rows, K, xq, xd, xsum, ks, ws, ts);
     if (ks > 1) return sum_splits(pt, ks, rows, ws, st);
     return hipGetLastError();
@@ -1225,23 +1267,20 @@ static hipError_t launch_raw_tm(const PartTable& pt, int ntm, int ntn, int ks, c
 
 hipError_t launch_mmq_q5k_raw(PartTable pt, int rows, int K, const int8_t* xq, const float* xd,
                               const int32_t* xsum, hipStream_t st, int cus, float* ws, size_t ws_floats) {
-    const int tm = mmq_tile_rows(rows, K, ntotal(pt), true, ws ? ws_floats : 0, 1.33f, true, cus);
+    const auto [tm, ks, ts] = mmq_pick(rows, K, ntotal(pt), true, ws ? ws_floats : 0, kCostRaw, cus);
     const int ntm = (rows + tm - 1) / tm, ntn = ntile_count(pt);
     if (ntm == 0 || ntn == 0) return hipSuccess;
-    const int ks = mmq_ksplit(rows, K, ntotal(pt), true, ws ? ws_floats : 0, tm, cus);
-    const TailSplit ts = ks > 1 ? TailSplit{}
-                                : mmq_tail_split(ntm * ntn, K >> 7, ws ? ws_floats : 0, tm, tm == 32 ? 1.33f : 1.f, cus);
     if (tm == 32) return launch_raw_tm<32>(pt, ntm, ntn, ks, ts, rows, K, xq, xd, xsum, st, ws);
     return launch_raw_tm<128>(pt, ntm, ntn, ks, ts, rows, K, xq, xd, xsum, st, ws);
 }
 
 hipError_t launch_mmq_q6k(PartTable pt, int rows, int K, const int8_t* xq, const float* xd,
                           hipStream_t st, int cus, float* ws, size_t ws_floats) {
-    const int tm = mmq_tile_rows(rows, K, ntotal(pt), false, ws ? ws_floats : 0, 1.06f, false, cus);
+    const TilePick pk = mmq_pick(rows, K, ntotal(pt), false, ws ? ws_floats : 0, kCostQ6, cus);
+    const int tm = pk.tm, ks = pk.ks;
     const int ntm = (rows + tm - 1) / tm, ntn = ntile_count(pt);
     if (ntm == 0 || ntn == 0) return hipSuccess;
-    const int ks = mmq_ksplit(rows, K, ntotal(pt), false, ws ? ws_floats : 0, tm, cus);
-    const dim3 grid(mmq_grid(ntm, ntn).x, ks);
+    const dim3 grid = mmq_grid(ntm, ntn, ks);
     if (tm == 32)
         launch_kernel(k_mmq_q6k_dma<32>, grid, dim3(256), 0, st, pt, ntm, ntn, rows, K, xq, xd, ks, ws);
     else

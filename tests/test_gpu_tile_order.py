@@ -1,8 +1,9 @@
 """The prefill GEMMs' grouped tile order (bq_gemm.hip tile_at) at the sizes
 where it can go wrong: more token tiles than one round (24 of 32 tokens, 8 of
 128; below that the order is panel-major), a last panel group narrower than the
-others, a ragged last token tile, several parts, and launches whose leftover
-tiles run as K slices.  Every output
+others, a ragged last token tile, several parts, launches whose leftover tiles
+run as K slices, and launches split over K whose pieces the XCDs share unevenly
+(map_tile: ranges that start and end inside a tile).  Every output
 is compared with the oracle of its tier (helpers.check), so a tile that is
 skipped, written twice from another tile's operands, or summed into another
 tile's place shows."""
@@ -20,6 +21,9 @@ CASES = [
     ("q5k", 256, [896, 256], 1157),        # raw tier
     ("q6k_rep", 512, [1664], 1157),        # 13 panels: a last group of five
     ("q5k_rep", 512, [384], 801),          # 26 token tiles of 32, fewer panels than a group
+    ("q6k_rep", 1792, [1664], 70),         # K slices over 13 x 3 tiles
+    ("q5k_rep", 2560, [1408], 300),        # K slices over 11 x 10 tiles
+    ("q5k", 1280, [896, 256], 150),        # raw tier, K slices over 9 x 5 tiles
 ]
 
 
