@@ -907,6 +907,10 @@ BQ_DEV void q6_stage(const SmemQ6Stage<TM>& sb, f32x16 (&acc)[TileGeo<TM>::NT][T
         for (int nt = 0; nt < G::NT; ++nt)
 #pragma unroll
             for (int mt = 0; mt < G::MT; ++mt) {
+                // the 32-token tile (168 registers at three waves per SIMD) spills
+                // when the four unrolled groups are scheduled together: 3072 x 9216
+                // at 2048 rows 280 -> 271 us; the 128-token tile loses 1-3% with it
+                if constexpr (TM == 32) __builtin_amdgcn_sched_barrier(0);
                 const f32x32 zero32 = {0.f};
                 const f32x32 sc = __builtin_amdgcn_mfma_f32_32x32x1f32(wsv[nt], xsv[mt], zero32, 0, 0, 0);
                 // 16-value dots: |D| <= 16 * 32 * 127 < 2^22, so the biased
