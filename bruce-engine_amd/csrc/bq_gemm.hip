@@ -11,11 +11,11 @@
 //     group per instruction, so the per-group scale is applied once per MFMA).
 //     Each kernel also has a 32-token tile (4 waves of 32x32, three
 //     workgroups per CU), chosen per launch by a work estimate.
-//   * K advances in 128-value stages.  The raw tier stages a stage in LDS
-//     with a 144-byte row stride (128 codes + 16 B pad: 4-dword bank offset
-//     per row, conflict-free 128-bit reads) and prefetches the next stage into
-//     registers while the current one is computed; the W144 and Q6_K kernels
-//     copy stages with direct-to-LDS loads (below).
+//   * K advances in 128-value stages.  Tokens, W144 and Q6_K weights reach LDS
+//     with direct-to-LDS loads (below); raw Q5_K blocks are prefetched one stage
+//     ahead into registers and unpacked to LDS codes with a 144-byte row stride
+//     (128 codes + 16 B pad: 4-dword bank offset per row, conflict-free 128-bit
+//     reads).
 //   * The k order inside an MFMA operand is irrelevant to the sum as long as A
 //     and B use the same order, so each lane simply loads 16 contiguous bytes.
 //   * Scales are staged q-major (sWs[q][row]) so a lane's 4 consecutive
@@ -245,15 +245,58 @@ BQ_DEV void stage_units_2x2(f32x16 (&acc)[2][2], int lh, const MfmaCvt& cv, Load
     }
 }
 
-// LDS layout for one stage
+constexpr int kXS = 128;  // token row stride in LDS (bytes)
+
+// Direct-to-LDS 16-byte load: lane i's 16 bytes from gbase + voff land at
+// LDS address lds + 16 * i.  Issued through asm so that the compiler does not
+// treat LDS reads of the other stage buffer, or the min term's global loads,
+// as dependent on it (with __builtin_amdgcn_global_load_lds it waits for
+// vmcnt(0) before them: 9216 x 3072 at M = 512 / 2048 / 8192 took 75 / 202 /
+// 765 us against 66 / 198 / 750 us with this asm); the kernel orders the
+// copies itself (vmcnt(0) + barrier before a buffer is read).  An untracked
+// VMEM op can only make the compiler's own vmcnt waits stricter, never looser.
+// m0 is written here; the compiler warns that it reserves m0 and will not
+// preserve it around the asm, which is safe because no other instruction of
+// these kernels reads or writes m0 (LDS instructions do not on gfx9; the
+// kernels have no other direct-to-LDS loads, s_sendmsg, or relative register
+// indexing).  tests/test_isa_m0.py checks that on the built code object.
+BQ_DEV void dma16(const void* gbase, uint32_t voff, const void* lds) {
+    const uint32_t m0 = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)lds);
+    asm volatile("s_mov_b32 m0, %2\n\tglobal_load_lds_dwordx4 %0, %1"
+                 :
+                 : "v"(voff), "s"(gbase), "s"(m0)
+                 : "m0", "memory");
+}
+
+// ---------------------------------------------------------------------------
+// Raw Q5_K prefill GEMM (the k_gemm_mmq_q5k semantics above).
+//   * Tokens, xd and xsum of stage s + 1 go straight to the other of two LDS
+//     buffers while stage s is computed.  Holding them in registers instead (24
+//     more per lane over the whole stage) left the 128-token tile none for the
+//     matrix-core conversions of stage_units_2x2, and it converted its dots on
+//     the VALU, which bounds this kernel.  With both changes, and the unpacking
+//     below, 9216 x 3072 at 2048 rows 223 -> 202 us, 14336 x 2560 at 512 rows
+//     88 -> 74, 3072 x 9216 at 4096 rows 462 -> 410, 2560 x 7168 at 700 rows
+//     72 -> 63; the 32-token tile, which converted on the matrix core before,
+//     keeps its time (3072 x 3072 at 37 rows 16.8 / 17.0).
+//   * One copy of the stage body (the token buffer picked by index): unrolled by
+//     two the 128-token tile spills.
+//   * Measured and not taken: the weight codes double-buffered too (80 KB, one
+//     barrier a stage): 3 registers spilled, 2-4% slower.
+// ---------------------------------------------------------------------------
+constexpr int kWP = 160;  // scale row stride [q][row]: the two lane halves' groups 32 banks apart
+
 template <int TM>
-struct Smem {
-    uint8_t w[kTN * kRS];      // weight codes, row stride 144
-    uint8_t x[TM * kRS];       // token codes, row stride 144
-    float ws[4 * kTN];         // ds   [q][row]
-    float xs[4 * TM];          // xd   [q][tok]
-    float wm[4 * kTN];         // raw: dmin*m      [q][row]
-    float xm[4 * TM];          // raw: -(xd*xsum)  [q][tok]
+struct SmemRawTok {
+    uint8_t x[TM * kXS];   // token codes, swizzled 16-byte slots
+    float xd[TM * 4];      // [tok][q]
+    int32_t xsum[TM * 4];  // [tok][q]
+};
+
+struct SmemRawW {
+    uint8_t w[kTN * kRS];  // weight codes, row stride 144
+    float ws[4 * kWP];     // ds      [q][row]
+    float wm[4 * kWP];     // dmin*m  [q][row]
 };
 
 template <int TM>
@@ -262,7 +305,8 @@ k_mmq_q5k_raw(PartTable pt, int ntm, int ntn, int rows, int K, const int8_t* __r
               const float* __restrict__ xd, const int32_t* __restrict__ xsum, int ksplit,
               float* __restrict__ part, TailSplit ts) {
     using G = TileGeo<TM>;
-    __shared__ __attribute__((aligned(16))) Smem<TM> sm;
+    __shared__ __attribute__((aligned(16))) SmemRawW sw;
+    __shared__ __attribute__((aligned(16))) SmemRawTok<TM> st[2];
     TileMap tm;
     int kc, left;
     if (!map_tile_tail<TM>(blockIdx.x, ntm, ntn, ts, tm, kc, ksplit, left)) return;
@@ -275,7 +319,8 @@ k_mmq_q5k_raw(PartTable pt, int ntm, int ntn, int rows, int K, const int8_t* __r
     // K split (slice kc of ksplit): stages [s0, s1) of this slice
     const int s0 = kc * nst / ksplit, s1 = (kc + 1) * nst / ksplit;
 
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int n0 = (wave / G::WM) * G::NT * 32, t0 = (wave % G::WM) * G::MT * 32;
     const int l32 = lane & 31, lh = lane >> 5;
 
@@ -287,162 +332,155 @@ k_mmq_q5k_raw(PartTable pt, int ntm, int ntn, int rows, int K, const int8_t* __r
 #pragma unroll
             for (int r = 0; r < 16; ++r) acc[a][b][r] = 0.f;
 
-    // ---- register prefetch of one stage -------------------------------------
-    // tokens: 8 TM chunks of 16 B (tok = c >> 3, part = c & 7), TM / 32 per
-    // thread; token scales: threads 0..TM-1 load xd[tok][4s..4s+3] and xsum.
-    u32x4 px[TM / 32];
-    f32x4 pxd;
-    i32x4 pxs;
-    // weights, raw: thread -> (row = tid >> 1, 64-value half hv = tid & 1)
+    // tokens of stage s: copied straight to LDS (codes 8 tokens per
+    // instruction, scales and sums 64; rows past `rows` keep stale bytes, their
+    // outputs are never stored)
+    const uint32_t x_off = (uint32_t)(lane >> 3) * (uint32_t)K + 16u * (uint32_t)((lane & 7) ^ (lane >> 3));
+    const uint32_t s_off = (uint32_t)lane * (uint32_t)(nb * 4);
+    auto dma_stage = [&](SmemRawTok<TM>& t, int s) {
+        const int8_t* xs0 = xq + (size_t)m0 * K + 128 * s;
+#pragma unroll
+        for (int i = 0; i < TM / 32; ++i) {
+            const int c = wave + 4 * i;
+            if (m0 + 8 * c + (lane >> 3) < rows) dma16(xs0 + (size_t)(8 * c) * K, x_off, t.x + 1024 * c);
+        }
+        constexpr int kSW = (TM + 63) / 64;  // waves that copy xd; as many copy xsum
+        if (wave < 2 * kSW) {
+            const int h = wave % kSW, tok = 64 * h + lane;
+            const size_t o = (size_t)(m0 + 64 * h) * nb + 4 * s;
+            const void* src = wave < kSW ? (const void*)(xd + o) : (const void*)(xsum + o);
+            const void* dst = wave < kSW ? (const void*)(t.xd + 256 * h) : (const void*)(t.xsum + 256 * h);
+            if (tok < TM && m0 + tok < rows) dma16(src, s_off, dst);
+        }
+    };
+
+    // weights: prefetched one stage ahead into registers, unpacked to LDS;
+    // thread -> (row = tid >> 1, 64-value half hv = tid & 1)
     u32x4 rqs0, rqs1, rqh0, rqh1, rhdr;
-
+    const int wrow = tid >> 1, hv = tid & 1;
     auto load_stage = [&](int s) {
-#pragma unroll
-        for (int i = 0; i < TM / 32; ++i) {
-            const int c = tid + 256 * i, tok = c >> 3, part = c & 7;
-            const int m = m0 + tok;
-            if (m < rows) px[i] = ld16(xq + (size_t)m * K + 128 * s + 16 * part);
-            else px[i] = (u32x4){0, 0, 0, 0};
-        }
-        if (tid < TM) {
-            const int m = m0 + tid;
-            if (m < rows) {
-                pxd = *(const f32x4*)(xd + (size_t)m * nb + 4 * s);
-                pxs = *(const i32x4*)(xsum + (size_t)m * nb + 4 * s);
-            } else {
-                pxd = (f32x4){0.f, 0.f, 0.f, 0.f};
-                pxs = (i32x4){0, 0, 0, 0};
-            }
-        }
-        {
-            const int row = tid >> 1, hv = tid & 1;
-            const uint8_t* blk = W + ((size_t)(nbase + row) * nsb + (s >> 1)) * kQ5Bytes;
-            const int j0 = 4 * (s & 1) + 2 * hv;  // sub-blocks j0, j0 + 1
-            rhdr = ld16(blk);
-            rqh0 = ld16(blk + 16);
-            rqh1 = ld16(blk + 32);
-            rqs0 = ld16(blk + 48 + 32 * (j0 >> 1));
-            rqs1 = ld16(blk + 64 + 32 * (j0 >> 1));
-        }
+        const uint8_t* blk = W + ((size_t)(nbase + wrow) * nsb + (s >> 1)) * kQ5Bytes;
+        const int j0 = 4 * (s & 1) + 2 * hv;  // sub-blocks j0, j0 + 1
+        rhdr = ld16(blk);
+        rqh0 = ld16(blk + 16);
+        rqh1 = ld16(blk + 32);
+        rqs0 = ld16(blk + 48 + 32 * (j0 >> 1));
+        rqs1 = ld16(blk + 64 + 32 * (j0 >> 1));
     };
-
     auto store_stage = [&](int s) {
+        const int j0 = 4 * (s & 1) + 2 * hv;
+        // codes of sub-blocks j0 (low nibbles) and j0+1 (high nibbles), 32 each:
+        // rotating qh by j - 4 puts the fifth bit at its place, so a dword takes
+        // a rotate, a bit select and a mask (and the high nibbles' shift)
+        u32x4 lo0, lo1, hi0, hi1;
+        const int sh = j0 + 28;  // alignbit takes the low five bits
 #pragma unroll
-        for (int i = 0; i < TM / 32; ++i) {
-            const int c = tid + 256 * i, tok = c >> 3, part = c & 7;
-            *(u32x4*)(sm.x + tok * kRS + 16 * part) = px[i];
+        for (int i = 0; i < 4; ++i) {
+            const uint32_t f0 = __builtin_amdgcn_alignbit(rqh0[i], rqh0[i], sh);
+            const uint32_t f1 = __builtin_amdgcn_alignbit(rqh1[i], rqh1[i], sh);
+            const uint32_t g0 = __builtin_amdgcn_alignbit(rqh0[i], rqh0[i], sh + 1);
+            const uint32_t g1 = __builtin_amdgcn_alignbit(rqh1[i], rqh1[i], sh + 1);
+            constexpr uint32_t kLo = 0x0F0F0F0Fu, kFive = 0x1F1F1F1Fu;
+            lo0[i] = ((rqs0[i] & kLo) | (f0 & ~kLo)) & kFive;
+            lo1[i] = ((rqs1[i] & kLo) | (f1 & ~kLo)) & kFive;
+            hi0[i] = (((rqs0[i] >> 4) & kLo) | (g0 & ~kLo)) & kFive;
+            hi1[i] = (((rqs1[i] >> 4) & kLo) | (g1 & ~kLo)) & kFive;
         }
-        if (tid < TM) {
+        uint8_t* dst = sw.w + wrow * kRS + 64 * hv;
+        *(u32x4*)(dst + 0) = lo0;
+        *(u32x4*)(dst + 16) = lo1;
+        *(u32x4*)(dst + 32) = hi0;
+        *(u32x4*)(dst + 48) = hi1;
+        const float d = h2f(rhdr.x & 0xFFFF), dmin = h2f(rhdr.x >> 16);
 #pragma unroll
-            for (int q = 0; q < 4; ++q) sm.xs[q * TM + tid] = pxd[q];
-#pragma unroll
-            for (int q = 0; q < 4; ++q) sm.xm[q * TM + tid] = -(pxd[q] * (float)pxs[q]);
-        }
-        {
-            const int row = tid >> 1, hv = tid & 1;
-            const int j0 = 4 * (s & 1) + 2 * hv;
-            // codes of sub-blocks j0 (low nibbles) and j0+1 (high nibbles), 32 each
-            u32x4 lo0, lo1, hi0, hi1;
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                lo0[i] = (rqs0[i] & 0x0F0F0F0Fu) | (((rqh0[i] >> j0) & 0x01010101u) << 4);
-                lo1[i] = (rqs1[i] & 0x0F0F0F0Fu) | (((rqh1[i] >> j0) & 0x01010101u) << 4);
-                hi0[i] = ((rqs0[i] >> 4) & 0x0F0F0F0Fu) | (((rqh0[i] >> (j0 + 1)) & 0x01010101u) << 4);
-                hi1[i] = ((rqs1[i] >> 4) & 0x0F0F0F0Fu) | (((rqh1[i] >> (j0 + 1)) & 0x01010101u) << 4);
-            }
-            uint8_t* dst = sm.w + row * kRS + 64 * hv;
-            *(u32x4*)(dst + 0) = lo0;
-            *(u32x4*)(dst + 16) = lo1;
-            *(u32x4*)(dst + 32) = hi0;
-            *(u32x4*)(dst + 48) = hi1;
-            const float d = h2f(rhdr.x & 0xFFFF), dmin = h2f(rhdr.x >> 16);
-#pragma unroll
-            for (int e = 0; e < 2; ++e) {
-                uint32_t sc, mm;
-                q5k_scale_min(rhdr.y, rhdr.z, rhdr.w, j0 + e, sc, mm);
-                const int q = 2 * hv + e;
-                sm.ws[q * kTN + row] = d * (float)sc;
-                sm.wm[q * kTN + row] = dmin * (float)mm;
-            }
+        for (int e = 0; e < 2; ++e) {
+            uint32_t sc, mm;
+            q5k_scale_min(rhdr.y, rhdr.z, rhdr.w, j0 + e, sc, mm);
+            const int q = 2 * hv + e;
+            sw.ws[q * kWP + wrow] = d * (float)sc;
+            sw.wm[q * kWP + wrow] = dmin * (float)mm;
         }
     };
 
-    load_stage(s0);
     const MfmaCvt cv = mfma_cvt_init(lane);
-    for (int s = s0; s < s1; ++s) {
-        __syncthreads();  // everyone is done reading the previous stage
-        store_stage(s);
-        __syncthreads();
-        if (s + 1 < s1) load_stage(s + 1);
-
-        // Per group pair (q0, q0+1) and tile: the scale products ds[n] * xd[m]
-        // of both groups come from one fp32 outer-product MFMA (32x32x1, two
-        // blocks: lanes 0-31 feed group q0, lanes 32-63 group q0+1), so the
-        // VALU epilogue is one convert and one FMA per output and group.
+    auto compute = [&](const SmemRawTok<TM>& t) {
+        // this lane half's groups lh and lh + 2: scales, dmin*m and -(xd*xsum)
+        float2 ws2[G::NT], wm2[G::NT], xs2[G::MT], xm2[G::MT];
 #pragma unroll
-        for (int qp = 0; qp < 2; ++qp) {
-            i32x4 a[G::NT][2], b[G::MT][2];  // [tile][group of the pair]
-            float wsv[G::NT], xsv[G::MT];
+        for (int nt = 0; nt < G::NT; ++nt) {
+            const int o = lh * kWP + n0 + nt * 32 + l32;
+            ws2[nt] = make_float2(sw.ws[o], sw.ws[o + 2 * kWP]);
+            wm2[nt] = make_float2(sw.wm[o], sw.wm[o + 2 * kWP]);
+        }
+#pragma unroll
+        for (int mt = 0; mt < G::MT; ++mt) {
+            const int o = 4 * (t0 + mt * 32 + l32);
+            const f32x4 d4 = *(const f32x4*)(t.xd + o);
+            const i32x4 s4 = *(const i32x4*)(t.xsum + o);
+            xs2[mt] = make_float2(lh ? d4[1] : d4[0], lh ? d4[3] : d4[2]);
+            xm2[mt] = make_float2(-(xs2[mt].x * (float)(lh ? s4[1] : s4[0])), -(xs2[mt].y * (float)(lh ? s4[3] : s4[2])));
+        }
+        // exact fp32 min term of the stage's four groups: two K=2 MFMAs per tile
+#pragma unroll
+        for (int nt = 0; nt < G::NT; ++nt)
+#pragma unroll
+            for (int mt = 0; mt < G::MT; ++mt) {
+                acc[nt][mt] = __builtin_amdgcn_mfma_f32_32x32x2f32(wm2[nt].x, xm2[mt].x, acc[nt][mt], 0, 0, 0);
+                acc[nt][mt] = __builtin_amdgcn_mfma_f32_32x32x2f32(wm2[nt].y, xm2[mt].y, acc[nt][mt], 0, 0, 0);
+            }
+        auto load_ops = [&](PairOps<G::NT, G::MT>& o, int qp) {
 #pragma unroll
             for (int e = 0; e < 2; ++e) {
-                const int q = 2 * qp + e;
+                const int g = 2 * qp + e;
 #pragma unroll
                 for (int nt = 0; nt < G::NT; ++nt)
-                    a[nt][e] = *(const i32x4*)(sm.w + (n0 + nt * 32 + l32) * kRS + 32 * q + 16 * lh);
-#pragma unroll
-                for (int mt = 0; mt < G::MT; ++mt)
-                    b[mt][e] = *(const i32x4*)(sm.x + (t0 + mt * 32 + l32) * kRS + 32 * q + 16 * lh);
-            }
-#pragma unroll
-            for (int nt = 0; nt < G::NT; ++nt) wsv[nt] = sm.ws[(2 * qp + lh) * kTN + n0 + nt * 32 + l32];
-#pragma unroll
-            for (int mt = 0; mt < G::MT; ++mt) xsv[mt] = sm.xs[(2 * qp + lh) * TM + t0 + mt * 32 + l32];
-#pragma unroll
-            for (int nt = 0; nt < G::NT; ++nt)
+                    o.a[nt][e] = *(const i32x4*)(sw.w + (n0 + nt * 32 + l32) * kRS + 32 * g + 16 * lh);
 #pragma unroll
                 for (int mt = 0; mt < G::MT; ++mt) {
-                    const f32x32 zero32 = {0.f};
-                    const f32x32 sc = __builtin_amdgcn_mfma_f32_32x32x1f32(wsv[nt], xsv[mt], zero32, 0, 0, 0);
-#pragma unroll
-                    for (int e = 0; e < 2; ++e) {
-                        if constexpr (TM == 32) {
-                            // matrix-core conversion (mfma_cvt_neg): the 32-token
-                            // tile has the registers for it (M = 512: 94-96 ->
-                            // 90-91 us); the 128-token tile would spill
-                            const i32x16 dd =
-                                __builtin_amdgcn_mfma_i32_32x32x32_i8(a[nt][e], b[mt][e], cv.bias, 0, 0, 0);
-                            const f32x16 ff = mfma_cvt_neg(cv, dd);
-#pragma unroll
-                            for (int r = 0; r < 16; ++r)
-                                acc[nt][mt][r] = __builtin_fmaf(-sc[16 * e + r], ff[r], acc[nt][mt][r]);
-                        } else {
-                            const i32x16 zero = {0};
-                            const i32x16 dd = __builtin_amdgcn_mfma_i32_32x32x32_i8(a[nt][e], b[mt][e], zero, 0, 0, 0);
-#pragma unroll
-                            for (int r = 0; r < 16; ++r)
-                                acc[nt][mt][r] = __builtin_fmaf(sc[16 * e + r], (float)dd[r], acc[nt][mt][r]);
-                        }
-                    }
+                    const int tok = t0 + mt * 32 + l32;
+                    o.b[mt][e] = *(const i32x4*)(t.x + tok * kXS + 16 * ((2 * g + lh) ^ (tok & 7)));
                 }
-        }
-        {
-            // exact fp32 min term of the stage's four groups: two K=2 MFMAs per tile
+            }
+        };
+        if constexpr (G::NT * G::MT == 4) {
+            stage_units_2x2(acc, lh, cv, load_ops, [&](int qp, int nt, int mt, int) {
+                return make_float2(qp ? ws2[nt].y : ws2[nt].x, qp ? xs2[mt].y : xs2[mt].x);
+            });
+        } else {
 #pragma unroll
             for (int qp = 0; qp < 2; ++qp) {
-                const int q = 2 * qp + lh;
-                float a[G::NT], b[G::MT];
+                PairOps<1, 1> o;
+                load_ops(o, qp);
+                const f32x32 zf = {0.f};
+                const f32x32 sc = __builtin_amdgcn_mfma_f32_32x32x1f32(qp ? ws2[0].y : ws2[0].x,
+                                                                      qp ? xs2[0].y : xs2[0].x, zf, 0, 0, 0);
 #pragma unroll
-                for (int nt = 0; nt < G::NT; ++nt) a[nt] = sm.wm[q * kTN + n0 + nt * 32 + l32];
+                for (int e = 0; e < 2; ++e) {
+                    const i32x16 dd = __builtin_amdgcn_mfma_i32_32x32x32_i8(o.a[0][e], o.b[0][e], cv.bias, 0, 0, 0);
+                    const f32x16 ff = mfma_cvt_neg(cv, dd);
 #pragma unroll
-                for (int mt = 0; mt < G::MT; ++mt) b[mt] = sm.xm[q * TM + t0 + mt * 32 + l32];
-#pragma unroll
-                for (int nt = 0; nt < G::NT; ++nt)
-#pragma unroll
-                    for (int mt = 0; mt < G::MT; ++mt)
-                        acc[nt][mt] = __builtin_amdgcn_mfma_f32_32x32x2f32(a[nt], b[mt], acc[nt][mt], 0, 0, 0);
+                    for (int r = 0; r < 16; ++r)
+                        acc[0][0][r] = __builtin_fmaf(-sc[16 * e + r], ff[r], acc[0][0][r]);
+                }
             }
         }
-    }
+    };
+
+    auto stage = [&](int s, const SmemRawTok<TM>& cur, SmemRawTok<TM>& nxt) {
+        BQ_WAIT_VM(0);    // this wave's copies and weight registers of stage s
+        __syncthreads();  // everyone's; and everyone is done reading stage s - 1
+        store_stage(s);
+        __syncthreads();
+        if (s + 1 < s1) {
+            dma_stage(nxt, s + 1);
+            load_stage(s + 1);
+        }
+        compute(cur);
+    };
+    dma_stage(st[0], s0);
+    load_stage(s0);
+#pragma unroll 1
+    for (int s = s0; s < s1; ++s) stage(s, st[(s - s0) & 1], st[(s - s0 + 1) & 1]);
 
     // ---- epilogue: Y[m][n], lane owns token column l32, rows 8*rg + 4*lh + 0..3
     // K split: slice kc's partial sums go to part[kc][part p: rows x N[p]];
@@ -493,35 +531,12 @@ k_mmq_q5k_raw(PartTable pt, int ntm, int ntn, int rows, int K, const int8_t* __r
 //     fp32 MFMAs do not, so the outer product costs VALU time; a one-block-
 //     per-group variant with the MFMAs of the next unit issued ahead was slower.)
 // ---------------------------------------------------------------------------
-constexpr int kXS = 128;  // token row stride in LDS (bytes)
-
 template <int TM>
 struct SmemStage {
     uint8_t w[kTN * kW144];  // 18432 B: W144 rows verbatim
     uint8_t x[TM * kXS];     // token codes, swizzled 16-byte slots
     float xs[TM * 4];        // xd[tok][q]
 };
-
-// Direct-to-LDS 16-byte load: lane i's 16 bytes from gbase + voff land at
-// LDS address lds + 16 * i.  Issued through asm so that the compiler does not
-// treat LDS reads of the other stage buffer, or the min term's global loads,
-// as dependent on it (with __builtin_amdgcn_global_load_lds it waits for
-// vmcnt(0) before them: 9216 x 3072 at M = 512 / 2048 / 8192 took 75 / 202 /
-// 765 us against 66 / 198 / 750 us with this asm); the kernel orders the
-// copies itself (vmcnt(0) + barrier before a buffer is read).  An untracked
-// VMEM op can only make the compiler's own vmcnt waits stricter, never looser.
-// m0 is written here; the compiler warns that it reserves m0 and will not
-// preserve it around the asm, which is safe because no other instruction of
-// these kernels reads or writes m0 (LDS instructions do not on gfx9; the
-// kernels have no other direct-to-LDS loads, s_sendmsg, or relative register
-// indexing).  tests/test_isa_m0.py checks that on the built code object.
-BQ_DEV void dma16(const void* gbase, uint32_t voff, const void* lds) {
-    const uint32_t m0 = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)lds);
-    asm volatile("s_mov_b32 m0, %2\n\tglobal_load_lds_dwordx4 %0, %1"
-                 :
-                 : "v"(voff), "s"(gbase), "s"(m0)
-                 : "m0", "memory");
-}
 
 // One stage's DMA; every wave issues instructions c = wave + 4i.  Per-lane
 // offsets are loop invariant (token slot swizzle: tok & 7 == lane >> 3), the
@@ -1060,9 +1075,11 @@ constexpr float kTailMinSaving = 192.f;  // see mmq_tail_split
 //   start[tm] + stages per slice x c[tm] x load + 2.5 us if a sum launch follows,
 // c = us per 128-value stage and workgroup per CU of a full GPU.  load: the
 // workgroups of the busiest CU (per XCD, as they are dealt), with two corrections.
-// A CU that holds a single 128-token tile takes 1.05 (one wave per SIMD keeps
-// it nearly as busy as two), one that holds two no less than `pair` = 1.6
-// (W144, unsplit) to 1.9 loads' time; the 32-token tile 1.3 and 1.9.  With the
+// A CU that holds a single 128-token tile takes `lone` (1.05: one wave per SIMD
+// keeps it nearly as busy as two; 1.22 for the raw tier, whose two barriers and
+// unpacking per stage a second workgroup covers), one that holds two no less
+// than `pair` = 1.6 (W144, unsplit) to 1.9 loads' time; the 32-token tile 1.3
+// and 1.9.  With the
 // leftover-tile split the load is the split one.  Fitted to both heights at
 // every split, 9 shapes x 11 row counts (9216 / 14336 / 8704 x 2560 / 3072 and
 // 2560 x 4096 W144, raw 3072 x 4096, Q6_K 3072 x 9216 and 2560 x 7168; 16..2048
@@ -1072,13 +1089,13 @@ constexpr float kTailMinSaving = 192.f;  // see mmq_tail_split
 // 128 rows 66.3 -> 57.8 / 27.6 -> 24.5, 2560 x 4096 at 1536 rows 66.6 -> 58.1,
 // raw 3072 x 4096 at 300 rows 37.1 -> 32.9.
 struct TileCost {
-    float c128, c32, pair;
+    float c128, c32, lone, pair;
     bool tail;   // the kernel takes the leftover-tile split
     float e32;   // its 32-token tile's cost per output over the 128-token one's
 };
-constexpr TileCost kCostW144 = {1.40f, 0.425f, 1.62f, true, 1.115f};
-constexpr TileCost kCostRaw = {2.02f, 0.62f, 1.92f, true, 1.33f};
-constexpr TileCost kCostQ6 = {2.4f, 0.64f, 1.9f, false, 1.f};
+constexpr TileCost kCostW144 = {1.40f, 0.425f, 1.05f, 1.62f, true, 1.115f};
+constexpr TileCost kCostRaw = {1.74f, 0.61f, 1.22f, 1.78f, true, 1.38f};
+constexpr TileCost kCostQ6 = {2.4f, 0.64f, 1.05f, 1.9f, false, 1.f};
 constexpr float kSplitUs = 2.5f, kStartUs128 = 11.5f, kStartUs32 = 9.f;
 
 struct TilePick {
@@ -1093,7 +1110,7 @@ TilePick mmq_pick(int rows, int K, int ntot, bool stage_units, size_t ws_floats,
     for (const int tm : {128, 32}) {
         const int ntiles = ((rows + tm - 1) / tm) * (ntot / kTN);
         const int ksmax = mmq_ksplit(rows, K, ntot, stage_units, ws_floats, tm, cus);
-        const float lone = tm == 128 ? 1.05f : 1.3f;
+        const float lone = tm == 128 ? tc.lone : 1.3f;
         for (int k = 1; k <= ksmax; ++k) {
             const int per = (units + k - 1) / k;
             if ((units + per - 1) / per != k) continue;  // fewer slices have the same longest one
