@@ -525,8 +525,8 @@ k_mmq_q5k_raw(PartTable pt, int ntm, int ntn, int rows, int K, const int8_t* __r
 //     DMA of stage s+1 runs while stage s is computed, one barrier per stage.
 //   * Per group pair and 32x32 tile: two v_mfma_i32_32x32x32_i8 dots, the
 //     scale products ds[n]*xd[m] of both groups from one two-block fp32
-//     outer-product MFMA, then one convert + one FMA per output and group
-//     (the 128-token tile converts on the matrix core instead: mfma_cvt_neg).
+//     outer-product MFMA, the dots' conversion on the matrix core
+//     (mfma_cvt_neg), then one FMA per output and group.
 //     (Measured on gfx950: int8 and bf16 MFMAs overlap independent VALU work,
 //     fp32 MFMAs do not, so the outer product costs VALU time; a one-block-
 //     per-group variant with the MFMAs of the next unit issued ahead was slower.)
@@ -585,25 +585,27 @@ BQ_DEV void mmq144_ops(PairOps<TileGeo<TM>::NT, TileGeo<TM>::MT>& o, const SmemS
 
 // One stage.  Per group pair and tile: the scale products of both groups come
 // from one two-block fp32 outer-product MFMA (lanes 0-31 feed group 2qp,
-// lanes 32-63 group 2qp+1), the two dots from two int8 MFMAs, then one convert
-// and one FMA per output and group.  The next pair's operands are read from
-// LDS while this pair is computed.  n0 / t0: the wave's first weight row /
-// token in the tile.
+// lanes 32-63 group 2qp+1), the two dots from two int8 MFMAs onto the conversion
+// bias, their floats from two bf16 MFMAs (mfma_cvt_neg), then one FMA per output
+// and group.  Bound by VALU issue: 32 converts per pair on the VALU cost as much
+// as the FMAs (3072 x 4096 at 1000 rows, three workgroups per CU: 53.3 us, on
+// the matrix core 50.5), and the two pairs unrolled let one's MFMAs run under
+// the other's FMAs (48.8; 9216 x 3072 at 37 rows 18.25 / 17.6 / 17.45, 2560 x
+// 7168 at 200 rows 26.8 / 26.1 / 25.7).  168 registers, no spill.  n0 / t0: the wave's
+// first weight row / token in the tile.
 template <int TM>
 BQ_DEV void mmq144_stage(const SmemStage<TM>& sb, f32x16 (&acc)[TileGeo<TM>::NT][TileGeo<TM>::MT], int n0,
-                         int t0, int l32, int lh) {
+                         int t0, int l32, int lh, const MfmaCvt& cv) {
     using G = TileGeo<TM>;
     f32x4 wsq[G::NT], xsq[G::MT];  // the stage's four scales per weight row / token: one 16-byte read each
 #pragma unroll
     for (int nt = 0; nt < G::NT; ++nt) wsq[nt] = *(const f32x4*)(sb.w + (n0 + nt * 32 + l32) * kW144 + 128);
 #pragma unroll
     for (int mt = 0; mt < G::MT; ++mt) xsq[mt] = *(const f32x4*)(sb.xs + 4 * (t0 + mt * 32 + l32));
-    PairOps<G::NT, G::MT> cur;
-    mmq144_ops<TM>(cur, sb, 0, n0, t0, l32, lh);
-#pragma unroll 1
+#pragma unroll
     for (int qp = 0; qp < 2; ++qp) {
-        PairOps<G::NT, G::MT> nxt;
-        mmq144_ops<TM>(nxt, sb, 1, n0, t0, l32, lh);  // qp = 1: harmless reread
+        PairOps<G::NT, G::MT> cur;
+        mmq144_ops<TM>(cur, sb, qp, n0, t0, l32, lh);
         float wsv[G::NT], xsv[G::MT];
 #pragma unroll
         for (int t = 0; t < G::NT; ++t) wsv[t] = qp ? (lh ? wsq[t][3] : wsq[t][2]) : (lh ? wsq[t][1] : wsq[t][0]);
@@ -614,17 +616,16 @@ BQ_DEV void mmq144_stage(const SmemStage<TM>& sb, f32x16 (&acc)[TileGeo<TM>::NT]
 #pragma unroll
             for (int mt = 0; mt < G::MT; ++mt) {
                 const f32x32 zf = {0.f};
-                const i32x16 zi = {0};
                 const f32x32 sc = __builtin_amdgcn_mfma_f32_32x32x1f32(wsv[nt], xsv[mt], zf, 0, 0, 0);
-                const i32x16 d0 = __builtin_amdgcn_mfma_i32_32x32x32_i8(cur.a[nt][0], cur.b[mt][0], zi, 0, 0, 0);
-                const i32x16 d1 = __builtin_amdgcn_mfma_i32_32x32x32_i8(cur.a[nt][1], cur.b[mt][1], zi, 0, 0, 0);
+                const i32x16 d0 = __builtin_amdgcn_mfma_i32_32x32x32_i8(cur.a[nt][0], cur.b[mt][0], cv.bias, 0, 0, 0);
+                const i32x16 d1 = __builtin_amdgcn_mfma_i32_32x32x32_i8(cur.a[nt][1], cur.b[mt][1], cv.bias, 0, 0, 0);
+                const f32x16 f0 = mfma_cvt_neg(cv, d0), f1 = mfma_cvt_neg(cv, d1);
 #pragma unroll
                 for (int r = 0; r < 16; ++r) {
-                    acc[nt][mt][r] = __builtin_fmaf(sc[r], (float)d0[r], acc[nt][mt][r]);
-                    acc[nt][mt][r] = __builtin_fmaf(sc[16 + r], (float)d1[r], acc[nt][mt][r]);
+                    acc[nt][mt][r] = __builtin_fmaf(-sc[r], f0[r], acc[nt][mt][r]);
+                    acc[nt][mt][r] = __builtin_fmaf(-sc[16 + r], f1[r], acc[nt][mt][r]);
                 }
             }
-        cur = nxt;
     }
 }
 
@@ -655,7 +656,7 @@ BQ_DEV void mmq144_stage_units(const SmemStage<TM>& sb, f32x16 (&acc)[TileGeo<TM
         });
 }
 
-// The 128-token tile takes stage_units_2x2 (with its matrix-core conversions
+// The 128-token tile takes stage_units_2x2 (its matrix-core conversions
 // measured 1-2% faster than converts on the VALU at M = 2048 / 8192); the
 // 32-token tile has one tile per wave.
 template <int TM>
@@ -664,7 +665,7 @@ BQ_DEV void mmq144_stage_any(const SmemStage<TM>& sb, f32x16 (&acc)[TileGeo<TM>:
     if constexpr (TileGeo<TM>::NT * TileGeo<TM>::MT == 4)
         mmq144_stage_units<TM>(sb, acc, n0, t0, l32, lh, cv);
     else
-        mmq144_stage<TM>(sb, acc, n0, t0, l32, lh);
+        mmq144_stage<TM>(sb, acc, n0, t0, l32, lh, cv);
 }
 
 // Eight consecutive xdh values half(xd * xsum) of one token row.  The
@@ -1078,7 +1079,7 @@ constexpr float kTailMinSaving = 192.f;  // see mmq_tail_split
 // A CU that holds a single 128-token tile takes `lone` (1.05: one wave per SIMD
 // keeps it nearly as busy as two; 1.22 for the raw tier, whose two barriers and
 // unpacking per stage a second workgroup covers), one that holds two no less
-// than `pair` = 1.6 (W144, unsplit) to 1.9 loads' time; the 32-token tile 1.3
+// than `pair` = 1.7 (W144, unsplit) to 1.9 loads' time; the 32-token tile 1.3
 // and 1.9.  With the
 // leftover-tile split the load is the split one.  Fitted to both heights at
 // every split, 9 shapes x 11 row counts (9216 / 14336 / 8704 x 2560 / 3072 and
@@ -1093,7 +1094,7 @@ struct TileCost {
     bool tail;   // the kernel takes the leftover-tile split
     float e32;   // its 32-token tile's cost per output over the 128-token one's
 };
-constexpr TileCost kCostW144 = {1.40f, 0.425f, 1.05f, 1.62f, true, 1.115f};
+constexpr TileCost kCostW144 = {1.40f, 0.385f, 1.05f, 1.70f, true, 1.03f};
 constexpr TileCost kCostRaw = {1.74f, 0.61f, 1.22f, 1.78f, true, 1.38f};
 constexpr TileCost kCostQ6 = {2.4f, 0.64f, 1.05f, 1.9f, false, 1.f};
 constexpr float kSplitUs = 2.5f, kStartUs128 = 11.5f, kStartUs32 = 9.f;
