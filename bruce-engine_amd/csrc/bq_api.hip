@@ -16,6 +16,7 @@
 
 #include "../../include/bq.h"
 #include "bq_internal.hpp"
+#include "bq_mmq_plan.hpp"
 
 using namespace bq;
 
@@ -432,14 +433,7 @@ constexpr int kGemmBMmqMin = 9;
 
 size_t bq_gemm_workspace_bytes_cus(int rows, int K, int n_total, int cus) {
     if (rows <= 0 || K <= 0 || n_total <= 0 || cus <= 0) return 0;
-    // The largest split any tier or tile height takes for this shape: the
-    // caller sizes one workspace per shape before it knows which tier a call
-    // takes (the raw tier, which splits at 128-value stages, can take more
-    // slices than the W144 and Q6_K kernels, which split at 256).
-    const int ks = std::max(mmq_ksplit(rows, K, n_total, true, (size_t)-1, 128, cus),
-                            mmq_ksplit(rows, K, n_total, true, (size_t)-1, 32, cus));
-    const size_t split = ks > 1 ? (size_t)ks * rows * n_total * sizeof(float) : 0;
-    return std::max(split, mmq_tail_ws_floats(rows, K, n_total, cus) * sizeof(float));
+    return mmq_ws_floats(rows, K, n_total, cus) * sizeof(float);
 }
 
 size_t bq_gemm_workspace_bytes(int rows, int K, int n_total) {

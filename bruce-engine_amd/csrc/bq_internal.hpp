@@ -99,12 +99,9 @@ hipError_t launch_repack_q5k(const void* raw, int K, int N, void* w144, uint16_t
 hipError_t launch_repack_q6k(const void* raw, int K, int N, void* w160, hipStream_t st);
 
 // prefill GEMMs (128-row weight tiles, int8 MFMA).  ws / ws_floats: the K-split
-// workspace (nullptr: no split); mmq_ksplit gives the split a launch takes
-// (stage_units: the raw tier, which splits at 128-value stages; tm: the
-// token-tile height, 128 or the W144 kernel's 32).  cus: the CU count of the
-// device the launch runs on (the workgroup slots every split choice counts).
-int mmq_ksplit(int rows, int K, int ntot, bool stage_units, size_t ws_floats, int tm, int cus);
-size_t mmq_tail_ws_floats(int rows, int K, int ntot, int cus);  // workspace of the Q5_K leftover-tile split
+// workspace (nullptr: no split).  cus: the CU count of the device the launch
+// runs on (the workgroup slots every split choice counts).  The token-tile
+// height and the split a launch takes: bq_mmq_plan.hpp.
 hipError_t launch_mmq_q5k_raw(PartTable pt, int rows, int K, const int8_t* xq, const float* xd,
                               const int32_t* xsum, hipStream_t st, int cus, float* ws = nullptr,
                               size_t ws_floats = 0);
