@@ -40,95 +40,6 @@ constexpr int kRS = 144;   // LDS row stride (bytes)
 
 typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
 
-struct TileMap {
-    int mt, nt;  // token tile, weight-row tile (over concatenated parts)
-};
-
-// Order of the tiles: an XCD's resident workgroups (64 of the 128-token tiles,
-// 96 of the 32-token ones) run consecutive indices at about the same K stage,
-// so the fewer bytes of weight panels and token tiles those cover, the more of
-// every stage its 4 MB L2 serves.  With more token tiles than one such round
-// wants, the order walks G panels per token tile instead of all token tiles of
-// one panel: G = 8 at 128 tokens (64 indices = 8 panels x 8 token tiles of 18 +
-// 16 KB a stage; panel-major 8192 rows: 1 x 64, 1 MB of tokens a stage from
-// beyond the L2), G = 4 at 32 tokens (18 and 4 KB: 4 x 24).  Up to kRound token
-// tiles the panel-major order is already as compact (512 rows as 32-token tiles,
-// 14336 x 2560: 66.4 us, in groups of 8 70.1).  9216 x 3072 W144: 8192 rows
-// 642 -> 606 us, 2048 rows 166.6 -> 162.2 (G = 4 / 16 1-2% behind at 8192 rows).
-template <int TM>
-BQ_DEV void tile_at(int idx, int ntm, int ntn, TileMap& t) {
-    constexpr int G = TM == 32 ? 4 : 8, kRound = TM == 32 ? 24 : 8;
-    if (ntm <= kRound) {
-        t.mt = idx % ntm;
-        t.nt = idx / ntm;
-        return;
-    }
-    const int grp = idx / (G * ntm), first = grp * G;
-    const int width = min(G, ntn - first), r = idx - first * ntm;
-    t.mt = r / width;
-    t.nt = first + r % width;
-}
-
-// Block b of a launch of ntm x ntn tiles in ks K slices -> (tile, slice kc).
-// The ntiles * ks pieces, a tile's slices next to each other, are dealt to the
-// XCDs in equal contiguous ranges (block b runs on XCD b % 8), so an XCD holds
-// at most one piece more than another; inside an XCD the blocks go slice by
-// slice, so that the first slices, which hold the W144 min term, start first and
-// on a CU each (two of them on one CU: 7040 x 5120 at 41 rows 21.9 -> 28.5 us).
-// (With the slices on blockIdx.y each XCD took ceil(ntiles / 8) tiles times
-// ks: Q6_K 2560 x 7168 at 640 rows, 100 tiles x 5 slices, put 65 workgroups on an
-// XCD's 64 slots: 97 us, now 67.  No block of a range may be empty: with 7 empty
-// ones in front of 63 the same call took 93.)
-template <int TM>
-BQ_DEV bool map_tile(int b, int ntm, int ntn, int ks, TileMap& t, int& kc) {
-    const int n = ntm * ntn * ks, per = (n + kXcds - 1) / kXcds;
-    const int p0 = (b % kXcds) * per, p1 = min(p0 + per, n);
-    int j = b / kXcds;
-    kc = 0;
-    if (p0 + j >= p1) return false;
-    if (ks == 1) {
-        tile_at<TM>(p0 + j, ntm, ntn, t);
-        return true;
-    }
-    // the j-th piece of [p0, p1) in the order of (slice, tile)
-    const int lead = p0 % ks;
-    int first;
-    for (;; ++kc) {
-        first = p0 + (kc >= lead ? kc - lead : kc - lead + ks);
-        const int c = first < p1 ? (p1 - 1 - first) / ks + 1 : 0;
-        if (j < c) break;
-        j -= c;
-    }
-    tile_at<TM>(first / ks + j, ntm, ntn, t);
-    return true;
-}
-
-// Block -> (tile, slice, slices).  Returns false for a block with no work.
-// XCD-major over the whole tiles as map_tile; a leftover tile's k slices are
-// consecutive blocks.
-template <int TM>
-BQ_DEV bool map_tile_tail(int b, int ntm, int ntn, const TailSplit& ts, TileMap& t, int& kc, int& ks, int& left) {
-    left = -1;
-    if (ts.k <= 1) return map_tile<TM>(b, ntm, ntn, ks, t, kc);
-    if (b < ts.gridfull) {
-        const int per = ts.gridfull / kXcds;
-        const int idx = (b % kXcds) * per + b / kXcds;
-        if (idx >= ts.nfull) return false;
-        tile_at<TM>(idx, ntm, ntn, t);
-        kc = 0;
-        ks = 1;
-        return true;
-    }
-    const int j = b - ts.gridfull;
-    if (j >= ts.nleft * ts.k) return false;
-    left = j / ts.k;
-    kc = j % ts.k;
-    ks = ts.k;
-    const int idx = ts.nfull + left;
-    tile_at<TM>(idx, ntm, ntn, t);
-    return true;
-}
-
 // offset of slice kc, part p in the K-split workspace [slice][part][rows][N[part]]
 BQ_DEV size_t split_offset(const PartTable& pt, int p, int kc, int rows) {
     size_t ntot = 0, off = 0;

@@ -1,7 +1,7 @@
 // bq_mmq_plan.hpp -- which launch a prefill GEMM takes (token-tile height, K
-// split, leftover-tile split) and the workspace that choice can use.  Host
-// arithmetic on the shape alone, without HIP: tests/test_mmq_plan.py builds it
-// with the host compiler.
+// split, leftover-tile split), the workspace that choice can use, and which
+// tile and K slice each block of the launch computes.  Arithmetic on the shape
+// alone, without HIP: tests/test_mmq_plan.py builds it with the host compiler.
 #pragma once
 #include <stddef.h>
 
@@ -12,6 +12,12 @@ namespace bq {
 
 constexpr int kTN = 128;   // weight rows per tile
 constexpr int kXcds = 8;
+
+#ifdef __HIPCC__
+#define BQ_HD __host__ __device__ __forceinline__
+#else
+#define BQ_HD inline
+#endif
 
 // Leftover-tile K split.  A launch of T tiles on C CUs runs for as long as its
 // busiest CU, which gets ceil(T / C) tiles; with T = q * C + L (0 < L < C)
@@ -189,6 +195,120 @@ inline size_t mmq_ws_floats(int rows, int K, int ntot, int cus) {
                             mmq_ksplit(rows, ntot, kCostRaw.units(K), (size_t)-1, 32, cus));
     const size_t split = ks > 1 ? (size_t)ks * rows * ntot : 0;
     return std::max(split, mmq_tail_ws_floats(rows, K, ntot, cus));
+}
+
+// ---------------------------------------------------------------------------
+// Block -> tile and K slice.
+// ---------------------------------------------------------------------------
+struct TileMap {
+    int mt, nt;  // token tile, weight-row tile (over concatenated parts)
+};
+
+// v / d for v, d >= 0 and v + d < 2^21 (SMALL), without the ~40 dependent
+// instructions of the integer division: (v + 0.5) / d is at least 0.5 / d from
+// the next integer, and the float error is at most (v / d + 1) * 2^-22.
+template <bool SMALL>
+BQ_HD int tile_div(int v, int d) {
+    if (!SMALL) return v / d;
+#ifdef __HIP_DEVICE_COMPILE__
+    return (int)(((float)v + 0.5f) * __builtin_amdgcn_rcpf((float)d));
+#else
+    return (int)(((float)v + 0.5f) * (1.f / (float)d));
+#endif
+}
+
+// Order of the tiles: an XCD's resident workgroups (64 of the 128-token tiles,
+// 96 of the 32-token ones) run consecutive indices at about the same K stage,
+// so the fewer bytes of weight panels and token tiles those cover, the more of
+// every stage its 4 MB L2 serves.  With more token tiles than one such round
+// wants, the order walks G panels per token tile instead of all token tiles of
+// one panel: G = 8 at 128 tokens (64 indices = 8 panels x 8 token tiles of 18 +
+// 16 KB a stage; panel-major 8192 rows: 1 x 64, 1 MB of tokens a stage from
+// beyond the L2), G = 4 at 32 tokens (18 and 4 KB: 4 x 24).  Up to kRound token
+// tiles the panel-major order is already as compact (512 rows as 32-token tiles,
+// 14336 x 2560: 66.4 us, in groups of 8 70.1).  9216 x 3072 W144: 8192 rows
+// 642 -> 606 us, 2048 rows 166.6 -> 162.2 (G = 4 / 16 1-2% behind at 8192 rows).
+template <int TM, bool SMALL = false>
+BQ_HD void tile_at(int idx, int ntm, int ntn, TileMap& t) {
+    constexpr int G = TM == 32 ? 4 : 8, kRound = TM == 32 ? 24 : 8;
+    if (ntm <= kRound) {
+        t.nt = tile_div<SMALL>(idx, ntm);
+        t.mt = idx - t.nt * ntm;
+        return;
+    }
+    const int grp = tile_div<SMALL>(idx, G * ntm), first = grp * G;
+    const int width = ntn - first < G ? ntn - first : G, r = idx - first * ntm;
+    t.mt = tile_div<SMALL>(r, width);
+    t.nt = first + r - t.mt * width;
+}
+
+// Block b of a launch of ntm x ntn tiles in ks K slices -> (tile, slice kc).
+// The n = ntiles * ks pieces, a tile's slices next to each other, are dealt to
+// the XCDs in contiguous ranges of ceil(n / 8) (block b runs on XCD b % 8; the
+// last range is what is left).  Inside an XCD the blocks go slice by slice, so
+// that the first slices, which hold the W144 min term, start first and
+// on a CU each (two of them on one CU: 7040 x 5120 at 41 rows 21.9 -> 28.5 us).
+// (With the slices on blockIdx.y each XCD took ceil(ntiles / 8) tiles times
+// ks: Q6_K 2560 x 7168 at 640 rows, 100 tiles x 5 slices, put 65 workgroups on an
+// XCD's 64 slots: 97 us, now 67.  With 7 empty blocks in front of 63 the same
+// call took 93.)
+// Every workgroup computes this before its first load, so it is closed-form: a
+// loop over the slices with an integer division each took 0.4-1 us of every
+// split launch (raw 7168 x 2560 at 24 rows 13.4 us, now 12.3; Q6_K 2560 x 4096 at
+// 12 rows 11.1, now 10.5).
+template <int TM>
+BQ_HD bool map_tile(int b, int ntm, int ntn, int ks, TileMap& t, int& kc) {
+    const unsigned n = ntm * ntn * ks, x = (unsigned)b % kXcds;
+    const int j = (unsigned)b / kXcds;
+    const int per = (n + kXcds - 1) / kXcds, p0 = x * per, p1 = p0 + per < (int)n ? p0 + per : (int)n;
+    kc = 0;
+    if (j >= p1 - p0) return false;
+    if (ks == 1) {
+        tile_at<TM>(p0 + j, ntm, ntn, t);
+        return true;
+    }
+    // The range starts at slice `lead` of tile t0 and holds q or q + 1 pieces of
+    // each slice (q + 1: the r slices from `lead` on, cyclically).  i: the j-th
+    // piece in the order of (slice, tile), counted from slice `lead`; it is the
+    // m-th piece of slice lead + c.  (A split launch has at most 3 pieces per CU.)
+    const int len = p1 - p0, t0 = tile_div<true>(p0, ks), lead = p0 - t0 * ks;
+    const int q = tile_div<true>(len, ks), r = len - q * ks;
+    const int c0 = lead ? ks - lead : 0;  // slice 0
+    int i = j + c0 * q + (c0 < r ? c0 : r);
+    if (i >= len) i -= len;
+    const bool longer = i < r * (q + 1);
+    const int rest = longer ? i : i - r * (q + 1), d = longer ? q + 1 : q;
+    const int g = tile_div<true>(rest, d), c = longer ? g : r + g, m = rest - g * d;
+    const bool next = lead + c >= ks;  // the piece is in the tile after its slice's first one
+    kc = next ? lead + c - ks : lead + c;
+    tile_at<TM, true>(t0 + m + (next ? 1 : 0), ntm, ntn, t);
+    return true;
+}
+
+// Block -> (tile, slice, slices).  Returns false for a block with no work.
+// XCD-major over the whole tiles as map_tile; a leftover tile's k slices are
+// consecutive blocks.
+template <int TM>
+BQ_HD bool map_tile_tail(int b, int ntm, int ntn, const TailSplit& ts, TileMap& t, int& kc, int& ks, int& left) {
+    left = -1;
+    if (ts.k <= 1) return map_tile<TM>(b, ntm, ntn, ks, t, kc);
+    if (b < ts.gridfull) {
+        const int per = ts.gridfull / kXcds;
+        const int idx = (b % kXcds) * per + b / kXcds;
+        if (idx >= ts.nfull) return false;
+        tile_at<TM>(idx, ntm, ntn, t);
+        kc = 0;
+        ks = 1;
+        return true;
+    }
+    const int j = b - ts.gridfull;
+    if (j >= ts.nleft * ts.k) return false;
+    left = j / ts.k;
+    kc = j % ts.k;
+    ks = ts.k;
+    const int idx = ts.nfull + left;
+    tile_at<TM>(idx, ntm, ntn, t);
+    return true;
 }
 
 }  // namespace bq

@@ -3,7 +3,8 @@ split, leftover-tile split) on the CPU: it depends on the shape alone as long as
 the caller holds the workspace bq_gemm_workspace_bytes reserves.  Under the
 reserved size every launch must be the one an unlimited workspace gives, or
 equal calls would take another path (another summation order) once a larger
-workspace is at hand."""
+workspace is at hand.  And the deal of a launch's blocks: every tile and K slice
+once, in the order the kernels count on."""
 import ctypes
 import os
 import subprocess
@@ -26,6 +27,8 @@ def picker(tmp_path_factory):
     L.t_pick.argtypes, L.t_pick.restype = [I, I, I, I, S, I, P], None
     L.t_ws_floats.argtypes, L.t_ws_floats.restype = [I, I, I, I], S
     L.t_reserved_differs.argtypes, L.t_reserved_differs.restype = [I, I, I, I, I, P], ctypes.c_long
+    L.t_deal.argtypes, L.t_deal.restype = [I] * 6, I
+    L.t_div.argtypes, L.t_div.restype = [I, I, P], None
     return L
 
 
@@ -47,3 +50,29 @@ def test_reserved_workspace_of_short_raw_k(picker):
         under = list(out)
         picker.t_pick(RAW, rows, 768, N, ctypes.c_size_t(-1).value, CUS, out)
         assert under == list(out), (N, rows)
+
+
+@pytest.mark.parametrize("tm", [32, 128])
+def test_every_piece_once(picker, tm):
+    """Whole and K-split launches on both sides of the grouped order's limit
+    (24 / 8 token tiles), panel counts around the groups of 4 / 8."""
+    for ntm in (1, 2, 3, 5, 7, 8, 9, 13, 23, 24, 25, 31, 64):
+        for ntn in (1, 2, 3, 4, 5, 7, 8, 9, 11, 15, 16, 17, 56, 72, 73):
+            for ks in range(1, 9):
+                if ks == 1 or ntm * ntn * ks <= 3 * 304:
+                    assert picker.t_deal(tm, ntm, ntn, ks, 1, 0) == 0, (ntm, ntn, ks)
+
+
+@pytest.mark.parametrize("tm", [32, 128])
+def test_leftover_split_pieces(picker, tm):
+    for ntm, ntn in ((32, 25), (9, 72), (16, 72), (41, 13), (8, 67), (25, 21)):
+        left = ntm * ntn % CUS
+        for k in (2, 3, 4):
+            assert picker.t_deal(tm, ntm, ntn, 1, k, left) == 0, (ntm, ntn, k)
+
+
+def test_short_division(picker):
+    """tile_div<true> over what a split launch asks of it: up to 3 pieces per CU."""
+    first = (ctypes.c_int * 2)()
+    picker.t_div(4096, 1025, first)
+    assert first[0] == -1, list(first)
