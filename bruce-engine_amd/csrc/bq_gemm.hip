@@ -1001,7 +1001,9 @@ static hipError_t launch_w144_tm(const PartTable& pt, int ntm, int ntn, int ks, 
 hipError_t launch_mmq_q5k_144(PartTable pt, int rows, int K, const int8_t* xq, const float* xd,
                               const int32_t* xsum, uint16_t* xdh, hipStream_t st, int cus, float* ws,
                               size_t ws_floats) {
-    const auto [tm, ks, ts] = mmq_pick(rows, K, ntotal(pt), ws ? ws_floats : 0, kCostW144, cus);
+    const TilePick pk = mmq_pick(rows, K, ntotal(pt), ws ? ws_floats : 0, kCostW144, cus);
+    const int tm = pk.tm, ks = pk.ks;
+    const TailSplit& ts = pk.ts;
     const int ntm = (rows + tm - 1) / tm;
     const int ntn = ntile_count(pt);
     if (ntm == 0 || ntn == 0) return hipSuccess;
@@ -1030,7 +1032,9 @@ static hipError_t launch_raw_tm(const PartTable& pt, int ntm, int ntn, int ks, c
 
 hipError_t launch_mmq_q5k_raw(PartTable pt, int rows, int K, const int8_t* xq, const float* xd,
                               const int32_t* xsum, hipStream_t st, int cus, float* ws, size_t ws_floats) {
-    const auto [tm, ks, ts] = mmq_pick(rows, K, ntotal(pt), ws ? ws_floats : 0, kCostRaw, cus);
+    const TilePick pk = mmq_pick(rows, K, ntotal(pt), ws ? ws_floats : 0, kCostRaw, cus);
+    const int tm = pk.tm, ks = pk.ks;
+    const TailSplit& ts = pk.ts;
     const int ntm = (rows + tm - 1) / tm, ntn = ntile_count(pt);
     if (ntm == 0 || ntn == 0) return hipSuccess;
     if (tm == 32) return launch_raw_tm<32>(pt, ntm, ntn, ks, ts, rows, K, xq, xd, xsum, st, ws);

@@ -36,165 +36,137 @@ struct TailSplit {
 
 // K split.  A launch with fewer tiles than the workgroup slots (two per CU
 // for the 128-token tiles, three for the 32-token tiles; 512 / 768 on
-// MI355X's 256 CUs) leaves CUs idle (one
-// token tile of a 9216-row matrix: 72 tiles), so it
-// is split over K into up to kMaxKSplit slices of whole K units (stage pairs
-// for the DMA-staged kernels, stages for the raw tier) when the caller's
-// workspace holds the slices' partial outputs [slice][part][rows][N[part]];
-// one more launch sums them in a fixed order.  The choice depends only on the
-// shape and the workspace size, so equal calls take equal paths (eager or
-// captured in a graph) and give equal bits.
-constexpr int kMaxKSplit = 8;
+// MI355X's 256 CUs) leaves CUs idle (one token tile of a 9216-row matrix: 72
+// tiles), so it may be split over K into up to kMaxKSplit slices of whole K
+// units (stage pairs for the DMA-staged kernels, stages for the raw tier) when
+// the caller's workspace holds the slices' partial outputs
+// [slice][part][rows][N[part]]; one more launch sums them in a fixed order.  The
+// choice depends only on the shape and the workspace size, so equal calls take
+// equal paths (eager or captured in a graph) and give equal bits.
+//
+// Leftover-tile split: k = 2 .. kMaxTailSplit slices per leftover tile, if that
+// takes at least half a tile off the busiest CU's ceil(tiles / CUs).  Measured
+// (9216 x 3072 W144, eager launches, us, unsplit -> split): 2048 rows (k = 2,
+// 0.5 tile) 181.5 -> 168.5; smaller gains did not pay for the shorter slices and
+// the summing launch (2560 rows, k = 3 for 0.33 tile: 216 -> 218), nor did more
+// than 4 slices (2304 rows, k = 8: 220 -> 227).  With one whole tile per CU each
+// runs alone on its CU and the leftover slices lose (512 x 9216 W144, 128-token
+// tiles: 62 -> 67 us).
+constexpr int kMaxKSplit = 8, kMaxTailSplit = 4;
 
-// `units`: the launch's slice units (TileCost::units).  `cus` below: the CU
-// count of the device the launch runs on (MI355X: 256), which sets the workgroup slots every split and tile-height choice counts.
-inline int mmq_ksplit(int rows, int ntot, int units, size_t ws_floats, int tm, int cus) {
-    const int ntiles = ((rows + tm - 1) / tm) * (ntot / kTN);
-    if (ntiles <= 0) return 1;
-    const int slots = (tm == 32 ? 3 : 2) * cus;  // workgroups resident at once (3 or 2 per CU)
-    int ks = std::min(kMaxKSplit, std::max(1, slots / ntiles));
-    while (ks > 1 && ((size_t)ks * rows * ntot > ws_floats || units < ks)) --ks;
-    // the fewest slices with the same longest slice (fewer partial outputs)
-    const int per = (units + ks - 1) / ks;
-    return (units + per - 1) / per;
-}
-
-// The leftover-tile split for `ntiles` tiles of `tm` tokens whose K has
-// `units` slice units: the k (2..4) that minimises the busiest CU's work,
-// floor(ntiles / CUs) + ceil(nleft * k / CUs) / k tiles, if that beats the
-// unsplit ceil(ntiles / CUs) by at least half a tile and the slices fit the
-// workspace; else k = 1.  Measured (9216 x 3072 W144, eager launches, µs,
-// unsplit -> split): 2048 rows (k = 2, 0.5 tile) 181.5 -> 168.5; smaller
-// gains did not pay for the shorter slices and the summing launch (2560 rows,
-// k = 3 for 0.33 tile: 216 -> 218), nor did more than 4 slices (2304 rows,
-// k = 8: 220 -> 227).
-// It must also save at least kTailMinSaving tile-token-units (tm x K units x
-// e, e = the tile height's relative cost per output) on the busiest CU, about
-// half of what the summing launch and the partial tiles cost.
-constexpr int kMaxTailSplit = 4;
-constexpr float kTailMinSaving = 192.f;
-inline TailSplit mmq_tail_split(int ntiles, int units, size_t ws_floats, int tm, float e, int cus) {
-    TailSplit ts;
-    const int q = ntiles / cus, nleft = ntiles % cus;
-    // with one whole tile per CU each runs alone on its CU and the leftover
-    // slices lose (512 x 9216 W144, 128-token tiles: 62 -> 67 us)
-    if (q < 2 || nleft == 0) return ts;
-    float best = (float)(q + 1);
-    int bk = 1;
-    for (int k = 2; k <= std::min(kMaxTailSplit, units); ++k) {
-        if ((size_t)nleft * k * kTN * tm > ws_floats) break;
-        const float load = (float)q + (float)((nleft * k + cus - 1) / cus) / (float)k;
-        if (load < best - 1e-6f) {
-            best = load;
-            bk = k;
-        }
-    }
-    if (bk == 1 || best > (float)(q + 1) - 0.5f) return ts;
-    if (((float)(q + 1) - best) * (float)tm * (float)units * e < kTailMinSaving) return ts;
-    ts.k = bk;
-    ts.nleft = nleft;
-    ts.nfull = ntiles - nleft;
-    ts.gridfull = (ts.nfull + kXcds - 1) / kXcds * kXcds;
-    return ts;
-}
-
-// Token-tile height (128 or 32) and K split of a launch: the pair with the
-// smallest estimated time
-//   start[tm] + stages per slice x c[tm] x load + 2.5 us if a sum launch follows,
-// c = us per 128-value stage and workgroup per CU of a full GPU.  load: the
-// workgroups of the busiest CU (per XCD, as they are dealt), with two corrections.
-// A CU that holds a single 128-token tile takes `lone` (1.05: one wave per SIMD
-// keeps it nearly as busy as two; 1.22 for the raw tier, whose two barriers and
-// unpacking per stage a second workgroup covers), one that holds two no less
-// than `pair` = 1.7 (W144, unsplit) to 1.9 loads' time; the 32-token tile 1.3
-// and 1.9.  With the
-// leftover-tile split the load is the split one.  Fitted to both heights at
-// every split, 9 shapes x 11 row counts (9216 / 14336 / 8704 x 2560 / 3072 and
-// 2560 x 4096 W144, raw 3072 x 4096, Q6_K 3072 x 9216 and 2560 x 7168; 16..2048
-// rows).  Against the estimate this replaces (tile height weighted by 1.06 ..
-// 1.33, always the largest split): 14336 x 2560 at 512 rows 68.1 -> 59.7 us
-// (128 tokens instead of 32), 9216 x 3072 at 768 rows 78.8 -> 69.2, 8704 x 2560 at 768 /
-// 128 rows 66.3 -> 57.8 / 27.6 -> 24.5, 2560 x 4096 at 1536 rows 66.6 -> 58.1,
-// raw 3072 x 4096 at 300 rows 37.1 -> 32.9.
+// Cost of one 128-value stage of a tile, us per workgroup and CU of a full GPU
+// (c128, c32: by tile height), and the W144 tier's min term, which is part of an
+// unsplit tile's cost and all in the first slice of a split one: w less per
+// stage there, and min_us per stage of the whole K.
 struct TileCost {
-    float c128, c32, lone, pair;
+    float c128, c32;
+    float w128, w32, min_us;
     bool stage_units;  // slices at 128-value stages (else at stage pairs)
     bool tail;         // the kernel takes the leftover-tile split
-    float e32;         // its 32-token tile's cost per output over the 128-token one's
     constexpr int units(int K) const { return stage_units ? K >> 7 : K >> 8; }
 };
-constexpr TileCost kCostW144 = {1.40f, 0.385f, 1.05f, 1.70f, false, true, 1.03f};
-constexpr TileCost kCostRaw = {1.74f, 0.61f, 1.22f, 1.78f, true, true, 1.38f};
-constexpr TileCost kCostQ6 = {2.4f, 0.64f, 1.05f, 1.9f, false, false, 1.f};
-constexpr float kSplitUs = 2.5f, kStartUs128 = 11.5f, kStartUs32 = 9.f;
+constexpr TileCost kCostW144 = {1.27f, 0.415f, 0.21f, 0.076f, 0.108f, false, true};
+constexpr TileCost kCostRaw = {1.60f, 0.623f, 0.f, 0.f, 0.f, true, true};
+constexpr TileCost kCostQ6 = {2.02f, 0.60f, 0.f, 0.f, 0.f, false, false};
 
+// A tile height: the workgroups a CU holds at once, us before the first stage
+// and after the last, and what a CU's last round costs, by its workgroups.
+struct TileHeight {
+    int tm, round;
+    float start, last[3];
+};
+constexpr TileHeight kTileHeights[2] = {{128, 2, 5.2f, {1.55f, 2.06f}}, {32, 3, 4.0f, {1.61f, 2.21f, 3.01f}}};
+constexpr float kSumUs = 2.3f, kSumTailUs = 4.4f, kPartialUs = 0.42e-6f;  // sum launches; per byte of partials
+
+// One launch a GEMM may take, what it writes to the workspace, and the
+// estimate of its time:
+//   start + stages per slice x c x load + (sum launch + its partials if split),
+// load = the workgroups of the busiest CU (as the XCDs are dealt) in whole rounds,
+// plus the last round's cost; with the leftover split its whole tiles + slices / k.
+// Fitted to the times of every height and split of 1512 shapes (9 .. 4096 rows, K
+// 768 .. 9216, N 512 .. 18432, all tiers; from 45 us on each launch repeated for
+// 12 ms, because the clock falls), minimising the time of the launch chosen: 0.8%
+// (W144), 0.4% (raw), 0.2% (Q6_K) over the fastest launch in the geometric mean.
+// The estimate it replaces, fitted to 9 shapes without a price on partials and
+// leftover sums, was 2.0 / 1.1 / 1.2% over it, and up to 15% slower than the one
+// before that: 9216 x 3072 W144 at 1279 rows 119.6 us (now 110.8), Q6_K 3200 x 8960
+// at 253 rows 57.0 (49.3), raw 6912 x 2048 at 247 rows 31.8 (26.5).  Over 640 other
+// shapes in turn W144 1.9, raw 3.2, Q6_K 2.6% faster (one 6%, four 3-4% slower).
 struct TilePick {
-    int tm, ks;
+    int tm = 128, ks = 1;
     TailSplit ts;
+    size_t ws_floats = 0;
+    float us = 0.f;
 };
 
-inline TilePick mmq_pick(int rows, int K, int ntot, size_t ws_floats, const TileCost& tc, int cus) {
-    TilePick best = {128, 1, {}};
-    float best_us = -1.f;
+// Calls f with every launch `rows` x ntot x K may take: both heights, every count
+// of slices with a longest slice of its own, every leftover split that saves more
+// than one of fewer slices.
+// `cus`: the CU count of the device the launch runs on (MI355X: 256).
+template <typename F>
+inline void mmq_launches(int rows, int K, int ntot, const TileCost& tc, int cus, F&& f) {
     const int units = tc.units(K);
-    for (const int tm : {128, 32}) {
-        const int ntiles = ((rows + tm - 1) / tm) * (ntot / kTN);
-        const int ksmax = mmq_ksplit(rows, ntot, units, ws_floats, tm, cus);
-        const float lone = tm == 128 ? tc.lone : 1.3f;
-        for (int k = 1; k <= ksmax; ++k) {
+    const float per_unit = tc.stage_units ? 1.f : 2.f;  // stages
+    for (const TileHeight& h : kTileHeights) {
+        const int tm = h.tm, ntiles = ((rows + tm - 1) / tm) * (ntot / kTN);
+        const float c = per_unit * (tm == 128 ? tc.c128 : tc.c32), w = per_unit * (tm == 128 ? tc.w128 : tc.w32);
+        const int ksmax = std::min({kMaxKSplit, units, h.round * cus / std::max(ntiles, 1)});
+        for (int k = 1; k <= std::max(ksmax, 1); ++k) {
             const int per = (units + k - 1) / k;
-            if ((units + per - 1) / per != k) continue;  // fewer slices have the same longest one
+            if (k > 1 && (units + per - 1) / per != k) continue;  // fewer slices have the same longest one
             const float l = (float)((ntiles * k + kXcds - 1) / kXcds) * (float)kXcds / (float)cus;
-            const float pair = tm == 128 && k == 1 ? tc.pair : 1.9f;
-            float load;
-            if (l <= 1.f)
-                load = lone;
-            else if (l <= 2.f)
-                load = std::max(l, pair);
-            else if (tm == 32)  // up to three at once, then one after another as slots free up
-                load = l <= 3.f ? 2.45f + 0.35f * (l - 2.f) : l + 0.3f;
-            else  // two at once: nearly whole rounds
-                load = std::min(std::ceil(l) + 0.05f, l + 0.6f);
-            TailSplit ts;
-            if (tc.tail && k == 1) ts = mmq_tail_split(ntiles, units, ws_floats, tm, tm == 32 ? tc.e32 : 1.f, cus);
-            if (ts.k > 1) load = (float)(ntiles / cus) + (float)((ts.nleft * ts.k + cus - 1) / cus) / (float)ts.k;
-            const float stage = (float)(tc.stage_units ? per : 2 * per) * (tm == 128 ? tc.c128 : tc.c32);
-            const float extra = k > 1 ? kSplitUs : 0.f;
-            const float us = (tm == 128 ? kStartUs128 : kStartUs32) + stage * load + extra;
-            if (best_us < 0.f || us < best_us) {
-                best_us = us;
-                best = {tm, k, ts};
-            }
+            const int full = std::max((int)std::ceil(l) - 1, 0);
+            const float load = (float)(full / h.round * h.round) + h.last[full % h.round];
+            TilePick p;
+            p.tm = tm;
+            p.ks = k;
+            p.ws_floats = k > 1 ? (size_t)k * rows * ntot : 0;
+            p.us = h.start + c * (float)per * load;
+            if (k > 1)
+                p.us += kSumUs + kPartialUs * 4.f * (float)p.ws_floats + per_unit * (float)units * tc.min_us -
+                        w * (float)per * load;
+            f(p);
+        }
+        const int q = ntiles / cus, nleft = ntiles % cus;
+        if (!tc.tail || q < 2 || nleft == 0) continue;
+        float least = 0.5f;  // of the leftover tile's time, on the busiest CU
+        for (int k = 2; k <= std::min(kMaxTailSplit, units); ++k) {
+            const float left = (float)((nleft * k + cus - 1) / cus) / (float)k;
+            if (k > 2 ? left >= least : left > least) continue;  // no more than fewer slices save
+            least = left;
+            TilePick p;
+            p.tm = tm;
+            p.ts.k = k;
+            p.ts.nleft = nleft;
+            p.ts.nfull = ntiles - nleft;
+            p.ts.gridfull = (p.ts.nfull + kXcds - 1) / kXcds * kXcds;
+            p.ws_floats = (size_t)nleft * k * kTN * tm;
+            p.us = h.start + c * (float)units * ((float)q + left) + kSumTailUs + kPartialUs * 4.f * (float)p.ws_floats;
+            f(p);
         }
     }
+}
+
+// The launch with the smallest estimate whose partial outputs fit the workspace.
+inline TilePick mmq_pick(int rows, int K, int ntot, size_t ws_floats, const TileCost& tc, int cus) {
+    TilePick best;
+    bool any = false;
+    mmq_launches(rows, K, ntot, tc, cus, [&](const TilePick& p) {
+        if (p.ws_floats > ws_floats || (any && p.us >= best.us)) return;
+        best = p;
+        any = true;
+    });
     return best;
 }
 
-// Workspace floats the leftover-tile split of either Q5_K tier takes for this
-// shape (the larger of the two tile heights), from the constants the launches
-// use, so that a launch under the reserved workspace is the one it takes under
-// any larger one.
-inline size_t mmq_tail_ws_floats(int rows, int K, int ntot, int cus) {
-    size_t need = 0;
-    for (const int tm : {128, 32}) {
-        const int ntiles = ((rows + tm - 1) / tm) * (ntot / kTN);
-        for (const TileCost& tc : {kCostW144, kCostRaw}) {
-            const TailSplit ts = mmq_tail_split(ntiles, tc.units(K), (size_t)-1, tm, tm == 32 ? tc.e32 : 1.f, cus);
-            if (ts.k > 1) need = std::max(need, (size_t)ts.nleft * ts.k * kTN * tm);
-        }
-    }
-    return need;
-}
-
-// Workspace floats that allow the largest split any tier or tile height takes
-// for this shape: a caller sizes one workspace per shape before it knows which
-// tier a call takes (the raw tier, which splits at 128-value stages, can take
-// more slices than the W144 and Q6_K kernels, which split at 256).
+// Workspace floats of the largest launch any tier may take for this shape, so
+// that every launch under it is the one it takes under any larger workspace (a
+// caller sizes one workspace per shape before it knows which tier a call takes).
 inline size_t mmq_ws_floats(int rows, int K, int ntot, int cus) {
-    const int ks = std::max(mmq_ksplit(rows, ntot, kCostRaw.units(K), (size_t)-1, 128, cus),
-                            mmq_ksplit(rows, ntot, kCostRaw.units(K), (size_t)-1, 32, cus));
-    const size_t split = ks > 1 ? (size_t)ks * rows * ntot : 0;
-    return std::max(split, mmq_tail_ws_floats(rows, K, ntot, cus));
+    size_t need = 0;
+    for (const TileCost& tc : {kCostW144, kCostRaw, kCostQ6})
+        mmq_launches(rows, K, ntot, tc, cus, [&](const TilePick& p) { need = std::max(need, p.ws_floats); });
+    return need;
 }
 
 // ---------------------------------------------------------------------------

@@ -52,6 +52,31 @@ def test_reserved_workspace_of_short_raw_k(picker):
         assert under == list(out), (N, rows)
 
 
+# Launches measured at every height and split: the fastest one (token-tile height,
+# K slices, slices per leftover tile), its time, and the time of the launch an
+# estimate fitted to nine shapes took instead (us).
+MEASURED = [
+    # tier, K, N, rows, height, slices, leftover slices
+    (W144, 3072, 9216, 905, 128, 1, 4),     # 85.0, was 91.0
+    (W144, 3072, 9216, 1279, 128, 1, 1),    # 110.8, was 119.6
+    (W144, 4096, 3072, 3717, 128, 1, 1),    # 144.1, was 156.0
+    (W144, 6144, 16640, 1128, 128, 1, 1),   # 325.5, was 369.2
+    (W144, 7168, 2560, 3268, 128, 1, 4),    # 172.8, was 193.3
+    (W144, 2560, 14336, 1281, 128, 1, 1),   # 147.1, was 161.4
+    (RAW, 2048, 6912, 247, 32, 1, 1),       # 26.5, was 31.8
+    (Q6, 8960, 3200, 253, 32, 3, 1),        # 49.3, was 57.0
+    (Q6, 768, 9216, 3040, 128, 1, 1),       # 108.6, was 120.6
+    (Q6, 8448, 8320, 3266, 128, 1, 1),      # 999, was 1095
+]
+
+
+@pytest.mark.parametrize("tier,K,N,rows,tm,ks,tail", MEASURED)
+def test_measured_fastest_launch(picker, tier, K, N, rows, tm, ks, tail):
+    out = (ctypes.c_int * 4)()
+    picker.t_pick(tier, rows, K, N, picker.t_ws_floats(rows, K, N, CUS), CUS, out)
+    assert list(out)[:3] == [tm, ks, tail]
+
+
 @pytest.mark.parametrize("tm", [32, 128])
 def test_every_piece_once(picker, tm):
     """Whole and K-split launches on both sides of the grouped order's limit
