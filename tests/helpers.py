@@ -1,8 +1,18 @@
 """Seeded synthetic inputs shared by the tests (generated by the oracle's
 splitmix64/Box-Muller stream, so GPU and CPU paths see identical bytes)."""
+import ctypes
+import functools
+import os
+import subprocess
+import tempfile
+
 import numpy as np
 
 import oracle as O
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+CUS = 256  # MI355X
+W144, RAW, Q6 = 0, 1, 2  # the prefill GEMMs' tiers
 
 
 def weights(seed, N, K, qtype="q5k", std=0.02):
@@ -93,3 +103,32 @@ def check(oracle, y, ref, tol=1e-4, floor=1e-2, etol=1e-3, what=""):
     assert nw < tol, (what, nw)
     assert ew < etol, (what, ew)
     return nw, ew
+
+
+@functools.lru_cache(maxsize=None)
+def mmq_plan():
+    """The prefill GEMMs' launch choice and deal (bq_mmq_plan.hpp behind
+    tests/host/mmq_plan.cpp), built with the host compiler."""
+    tmp = tempfile.TemporaryDirectory()
+    so = os.path.join(tmp.name, "mmq_plan.so")
+    subprocess.run(["g++", "-std=c++17", "-O2", "-shared", "-fPIC", "-I",
+                    os.path.join(ROOT, "bruce-engine_amd", "csrc"), os.path.join(ROOT, "tests", "host", "mmq_plan.cpp"),
+                    "-o", so], check=True)
+    L = ctypes.CDLL(so)
+    I, S, P = ctypes.c_int, ctypes.c_size_t, ctypes.POINTER(ctypes.c_int)
+    L.t_pick.argtypes, L.t_pick.restype = [I, I, I, I, S, I, P], None
+    L.t_ws_floats.argtypes, L.t_ws_floats.restype = [I, I, I, I], S
+    L.t_reserved_differs.argtypes, L.t_reserved_differs.restype = [I, I, I, I, I, P], ctypes.c_long
+    L.t_deal.argtypes, L.t_deal.restype = [I] * 6, I
+    L.t_div.argtypes, L.t_div.restype = [I, I, P], None
+    return L
+
+
+def mmq_launch(tier, K, N, rows, ws_floats=None):
+    """(token-tile height, K slices, slices per leftover tile, leftover tiles) of
+    the launch a prefill GEMM takes on MI355X; ws_floats None: the reserved workspace."""
+    L = mmq_plan()
+    out = (ctypes.c_int * 4)()
+    ws = L.t_ws_floats(rows, K, N, CUS) if ws_floats is None else ws_floats
+    L.t_pick(tier, rows, K, N, ws, CUS, out)
+    return tuple(out)

@@ -401,8 +401,8 @@ def test_mmq_q5k_ragged_parts(bq, oracle, prepacked):
 
 
 # Row counts that are not multiples of either token tile, multi-part launches
-# with unequal N, and K-split classes: each case's tile height and split come
-# from the launch's work estimate (both heights occur below).
+# with unequal N, in K slices (97, 129 and 300 rows) and whole (1000 rows), all on
+# the 32-token tile; the 128-token tile's launches: test_gpu_tile_order.py.
 @pytest.mark.parametrize("prepacked", [False, True])
 @pytest.mark.parametrize("M,Ns,K", [(97, [256, 128], 1024), (129, [128, 384], 1536), (300, [256, 128, 128], 1024),
                                     (1000, [384], 512)])
@@ -511,8 +511,8 @@ def test_mmq_config4_full_slices(bq, oracle):
 
 @pytest.mark.parametrize("rows", [17, 100, 128])
 def test_mmq_w144_ksplit(bq, oracle, rows):
-    """The W144 GEMM over one token tile split into 8 K slices (3072 / 256 = 12
-    stage pairs; 8 weight-row tiles): against the oracle, and bit-identical
+    """The W144 GEMM over 1 to 4 token tiles split into 6 K slices (3072 / 256 =
+    12 stage pairs; 8 weight-row tiles): against the oracle, and bit-identical
     between two calls (the slices are summed in a fixed order)."""
     import torch
     K, N = 3072, 1024

@@ -6,30 +6,17 @@ equal calls would take another path (another summation order) once a larger
 workspace is at hand.  And the deal of a launch's blocks: every tile and K slice
 once, in the order the kernels count on."""
 import ctypes
-import os
-import subprocess
 
 import pytest
 
-ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
-W144, RAW, Q6 = 0, 1, 2
-CUS = 256  # MI355X
+import test_gpu_raw_stages
+import test_gpu_tile_order
+from helpers import CUS, Q6, RAW, W144, mmq_launch, mmq_plan
 
 
 @pytest.fixture(scope="module")
-def picker(tmp_path_factory):
-    so = tmp_path_factory.mktemp("mmq_plan") / "mmq_plan.so"
-    subprocess.run(["g++", "-std=c++17", "-O2", "-shared", "-fPIC", "-I",
-                    os.path.join(ROOT, "bruce-engine_amd", "csrc"), os.path.join(ROOT, "tests", "host", "mmq_plan.cpp"),
-                    "-o", str(so)], check=True)
-    L = ctypes.CDLL(str(so))
-    I, S, P = ctypes.c_int, ctypes.c_size_t, ctypes.POINTER(ctypes.c_int)
-    L.t_pick.argtypes, L.t_pick.restype = [I, I, I, I, S, I, P], None
-    L.t_ws_floats.argtypes, L.t_ws_floats.restype = [I, I, I, I], S
-    L.t_reserved_differs.argtypes, L.t_reserved_differs.restype = [I, I, I, I, I, P], ctypes.c_long
-    L.t_deal.argtypes, L.t_deal.restype = [I] * 6, I
-    L.t_div.argtypes, L.t_div.restype = [I, I, P], None
-    return L
+def picker():
+    return mmq_plan()
 
 
 @pytest.mark.parametrize("tier,k_step", [(W144, 512), (RAW, 256), (Q6, 256)])
@@ -72,9 +59,28 @@ MEASURED = [
 
 @pytest.mark.parametrize("tier,K,N,rows,tm,ks,tail", MEASURED)
 def test_measured_fastest_launch(picker, tier, K, N, rows, tm, ks, tail):
-    out = (ctypes.c_int * 4)()
-    picker.t_pick(tier, rows, K, N, picker.t_ws_floats(rows, K, N, CUS), CUS, out)
-    assert list(out)[:3] == [tm, ks, tail]
+    assert mmq_launch(tier, K, N, rows)[:3] == (tm, ks, tail)
+
+
+def test_measured_case_launches():
+    """The GPU tests of the tile order and of the raw tier's staging name the
+    launch each case is there for: the choice still takes it, and together they
+    run both heights of every tier whole and K-split and both of the Q5_K
+    tiers' leftover splits, each in the grouped order with a narrow last group."""
+    seen = set()
+    for fmt, K, Ns, rows, launch in test_gpu_tile_order.CASES:
+        tier = {"q5k_rep": W144, "q5k": RAW, "q6k_rep": Q6}[fmt]
+        tm, ks, tail, left = mmq_launch(tier, K, sum(Ns), rows)
+        assert (tm, ks, tail) == launch, (fmt, K, Ns, rows)
+        ntm, ntn, group, rnd = -(-rows // tm), sum(Ns) // 128, *((4, 24) if tm == 32 else (8, 8))
+        if ntm > rnd and ntn % group:
+            seen.add((tier, tm, "tail" if tail > 1 else "split" if ks > 1 else "whole"))
+            if tail > 1:  # leftover tiles inside the narrow group
+                assert left <= ntm * (ntn % group)
+    for K, N, rows, launch in test_gpu_raw_stages.CASES:
+        assert mmq_launch(RAW, K, N, rows)[:3] == launch, (K, N, rows)
+    want = {(t, tm, m) for t in (W144, RAW, Q6) for tm in (32, 128) for m in ("whole", "split", "tail")}
+    assert seen == want - {(Q6, 32, "tail"), (Q6, 128, "tail")}
 
 
 @pytest.mark.parametrize("tm", [32, 128])
