@@ -481,11 +481,13 @@ BQ_DEV void mmq144_ops(PairOps<TileGeo<TM>::NT, TileGeo<TM>::MT>& o, const SmemS
 // from one two-block fp32 outer-product MFMA (lanes 0-31 feed group 2qp,
 // lanes 32-63 group 2qp+1), the two dots from two int8 MFMAs onto the conversion
 // bias, their floats from two bf16 MFMAs (mfma_cvt_neg), then one FMA per output
-// and group.  Bound by VALU issue: 32 converts per pair on the VALU cost as much
-// as the FMAs (3072 x 4096 at 1000 rows, three workgroups per CU: 53.3 us, on
-// the matrix core 50.5), and the two pairs unrolled let one's MFMAs run under
-// the other's FMAs (48.8; 9216 x 3072 at 37 rows 18.25 / 17.6 / 17.45, 2560 x
-// 7168 at 200 rows 26.8 / 26.1 / 25.7).  168 registers, no spill.  n0 / t0: the wave's
+// and group.  Bound by the chain dot -> conversion -> FMA at three waves per SIMD,
+// not by issue: 9216 x 3072 at 512 rows has the VALU busy for 29% of the cycles and
+// the matrix core for 31%; with the converts on the VALU (18.2M instructions, now
+// 10.0M; 50% busy) it took 5% more cycles.  3072 x 4096 at 1000 rows: converts on
+// the VALU 53.3 us, on the matrix core 50.5, the two pairs unrolled, so that one's
+// MFMAs run under the other's FMAs, 48.8; 9216 x 3072 at 37 rows 18.25 / 17.6 /
+// 17.45, 2560 x 7168 at 200 rows 26.8 / 26.1 / 25.7.  168 registers, no spill.  n0 / t0: the wave's
 // first weight row / token in the tile.
 template <int TM>
 BQ_DEV void mmq144_stage(const SmemStage<TM>& sb, f32x16 (&acc)[TileGeo<TM>::NT][TileGeo<TM>::MT], int n0,
@@ -817,9 +819,10 @@ BQ_DEV void q6_stage(const SmemQ6Stage<TM>& sb, f32x16 (&acc)[TileGeo<TM>::NT][T
         for (int nt = 0; nt < G::NT; ++nt)
 #pragma unroll
             for (int mt = 0; mt < G::MT; ++mt) {
-                // the 32-token tile (168 registers at three waves per SIMD) spills
-                // when the four unrolled groups are scheduled together: 3072 x 9216
-                // at 2048 rows 280 -> 271 us; the 128-token tile loses 1-3% with it
+                // the 32-token tile (168 registers at three waves per SIMD) spills two
+                // registers when the four unrolled groups are scheduled together: 3072 x
+                // 9216 at 1000 rows 150.8 -> 149.2 us, 3072 x 4096 at 3000 196.7 -> 195.1,
+                // 60, 2048 and 8192 rows level; the 128-token tile loses 1-3% with it
                 if constexpr (TM == 32) __builtin_amdgcn_sched_barrier(0);
                 const f32x32 zero32 = {0.f};
                 const f32x32 sc = __builtin_amdgcn_mfma_f32_32x32x1f32(wsv[nt], xsv[mt], zero32, 0, 0, 0);

@@ -199,7 +199,8 @@ BQ_HD int tile_div(int v, int d) {
 // beyond the L2), G = 4 at 32 tokens (18 and 4 KB: 4 x 24).  Up to kRound token
 // tiles the panel-major order is already as compact (512 rows as 32-token tiles,
 // 14336 x 2560: 66.4 us, in groups of 8 70.1).  9216 x 3072 W144: 8192 rows
-// 642 -> 606 us, 2048 rows 166.6 -> 162.2 (G = 4 / 16 1-2% behind at 8192 rows).
+// 635.9 -> 600.6 us, 2048 rows 164.7 -> 161.6 (G = 4 / 16 1-2% behind at 8192
+// rows); bytes from beyond the L2s 2262 -> 741 MB and 202 -> 162 MB.
 template <int TM, bool SMALL = false>
 BQ_HD void tile_at(int idx, int ntm, int ntn, TileMap& t) {
     constexpr int G = TM == 32 ? 4 : 8, kRound = TM == 32 ? 24 : 8;
